@@ -9,7 +9,7 @@
 // and after the last layer k_resnorm(output_norm) -> k_gemv(head, softcap).
 #include "z2h.h"
 #include "z2h_kernels.h"
-#include "z2h_gemm.h"
+#include "z2h_gemm_q.h"
 #include "z2h_attn.h"
 #include <hip/hip_ext.h>
 #include "z2_formats.h"
@@ -35,6 +35,17 @@ extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, false, true>(
 extern template __global__ void k_gemv_split<WF_Q8_0, true, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, true, true>(GemvArgs);
+// the Q8_0 and Q6_K GEMMs, instantiated in z2h_wide.hip
+extern template __global__ void k_gemm_q80<true, 1>(GemmArgs);
+extern template __global__ void k_gemm_q80<true, 2>(GemmArgs);
+extern template __global__ void k_gemm_q80<false, 1>(GemmArgs);
+extern template __global__ void k_gemm_q80<false, 2>(GemmArgs);
+extern template __global__ void k_gemm_q6k<true, 1>(GemmArgs);
+extern template __global__ void k_gemm_q6k<true, 2>(GemmArgs);
+extern template __global__ void k_gemm_q6k<true, 4>(GemmArgs);
+extern template __global__ void k_gemm_q6k<false, 1>(GemmArgs);
+extern template __global__ void k_gemm_q6k<false, 2>(GemmArgs);
+extern template __global__ void k_gemm_q6k<false, 4>(GemmArgs);
 } // namespace z2d
 
 namespace {
@@ -603,14 +614,28 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 }
 
 // ---------------------------------------------------------------- launch helpers
-// Passes of more than 64 token rows (prefill chunks, mixed passes) run their Q4_K (m16) matmuls as
-// GEMMs (k_gemm_q4k), decode steps the GEMVs: both fold a row's superblocks in the same order with
-// the same operations. Every F16 (t64) matmul runs on k_gemm_f16, in its wide or narrow shape (same
-// bits per row either way).
+// Wide matmuls run as GEMMs, narrow ones as the decode GEMVs; both fold a row's blocks in the same order
+// with the same operations, so the lines below are about speed alone.
+//   F16 (t64)    always k_gemm_f16, in its wide or narrow shape (same bits per row either way).
+//   Q4_K (m16)   passes of more than 64 token rows (k_gemm_q4k's tile height).
+//   Q8_0, Q6_K   dense: more 16-row token tiles x row-group quads than half the compute units. Below that the
+//                K-split GEMV's four times as many blocks win (48 rows of QKV, 147 blocks: 8.0 us against 10.5
+//                for Q8_0; 64 rows of W_o, 128 blocks: 8.0 against 6.5; the 9225-row
+//                Q8_0 head of 5 rows 8.8 against 10.1, of 16 rows 9.7 against 12.5, of 64 rows 17.6 against
+//                27.4). One and two rows keep the token-pair units. Experts: at least 8 routes per expert
+//                on average, where the GEMV starts re-reading its weights per 8- or 16-route pass (64 rows,
+//                top-4 of 32: Q6_K gate/up 38 us against 52, down 22 against 32; 48 rows, 6 routes: level
+//                before the sort launch is counted).
 constexpr int GEMM_MIN_ROWS = 65;
-bool use_gemm(const DevMat & m, int n_tok) {
-    if (!m.m16 && m.type == Z2H_F16) return true;
-    return n_tok >= GEMM_MIN_ROWS && m.m16 && m.type == Z2H_Q4_K;
+bool use_gemm(const z2h_ctx * ctx, const DevMat & m, int n_tok) {
+    if (!m.m16) return m.type == Z2H_F16;
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
+    return n_tok > 2 && 2ll * ((m.tiles + 3) / 4) * ((n_tok + 15) / 16) > ctx->n_cu;
+}
+bool use_gemm_experts(const DevMat & m, int n_tok, int k, int E) {
+    if (!m.m16) return m.type == Z2H_F16;
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
+    return n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
 }
 // gate and up fused with SwiGLU in one GEMM launch: same type, layout and shape
 bool gemm_dual_ok(const DevMat & g, const DevMat & u) {
@@ -639,6 +664,26 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
         const dim3 grid(dual ? (m0.tiles + 3) / 4 : (m0.tiles + 7) / 8, gemm_slots(a.grouped, a.n_tok, a.k, a.E, GM_T));
         if (dual) KL(k_gemm_q4k<true>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
         else KL(k_gemm_q4k<false>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
+    } else if (m0.m16) {
+        // the tallest token tile that is half full on average and leaves at least two blocks per compute
+        // unit (grouped launches fill about routes / GT + E / 2 tile slots): 333 rows of Q8_0 W_o 11.0 us
+        // with 16-row tiles against 13.7 with 32, 1024 rows of QKV 50 against 36. Q8_0 stops at 32 rows:
+        // 64 halve the resident waves (1500 rows, top-4 of 32: gate/up 216 us against 176).
+        const int bx = (m0.tiles + 3) / 4, tmax = m0.type == Z2H_Q8_0 ? 2 : 4;
+        const int items = a.grouped ? a.n_tok * a.k : a.n_tok, per = a.grouped ? items / a.E : items;
+        int ts = tmax;
+        while (ts > 1 && (per < 8 * ts || (int64_t) bx * (a.grouped ? items / (16 * ts) + a.E / 2 : (items + 16 * ts - 1) / (16 * ts)) < 2 * ctx->n_cu)) ts >>= 1;
+        const dim3 grid(bx, gemm_slots(a.grouped, a.n_tok, a.k, a.E, 16 * ts));
+#define GQ(K_, D_, T_, L_) KL((K_<D_, T_>), grid, dim3(256), L_(T_), ctx->stream, a)
+        if (m0.type == Z2H_Q8_0) {
+            if (ts == 1) { if (dual) GQ(k_gemm_q80, true, 1, gemm_q80_lds); else GQ(k_gemm_q80, false, 1, gemm_q80_lds); }
+            else { if (dual) GQ(k_gemm_q80, true, 2, gemm_q80_lds); else GQ(k_gemm_q80, false, 2, gemm_q80_lds); }
+        } else {
+            if (ts == 1) { if (dual) GQ(k_gemm_q6k, true, 1, gemm_q6k_lds); else GQ(k_gemm_q6k, false, 1, gemm_q6k_lds); }
+            else if (ts == 2) { if (dual) GQ(k_gemm_q6k, true, 2, gemm_q6k_lds); else GQ(k_gemm_q6k, false, 2, gemm_q6k_lds); }
+            else { if (dual) GQ(k_gemm_q6k, true, 4, gemm_q6k_lds); else GQ(k_gemm_q6k, false, 4, gemm_q6k_lds); }
+        }
+#undef GQ
     } else {
         // wide tiles (64 token rows) for wide dense passes and experts averaging 32+ routes, else
         // narrow ones (16 token rows, 16 output rows per wave)
@@ -667,7 +712,7 @@ bool xf_split_ok(const z2h_ctx * ctx, const DevMat & m, int rows, bool grouped) 
 }
 
 int launch_gemv(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvArgs & base, int grid_y, int fam) {
-    if (use_gemm(m0, base.n_tok) && (!m1 || gemm_dual_ok(m0, *m1)) && (!base.grouped || (base.r_off && base.r_perm)))
+    if ((base.grouped ? use_gemm_experts(m0, base.n_tok, base.k, base.E) : use_gemm(ctx, m0, base.n_tok)) && (!m1 || gemm_dual_ok(m0, *m1)) && (!base.grouped || (base.r_off && base.r_perm)))
         return launch_gemm(ctx, m0, m1, base, fam);
     prof_scope ps(ctx, fam);
     GemvArgs a = base;
@@ -787,11 +832,11 @@ int launch_gemv(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
     return Z2H_OK;
 }
 
-// SwiGLU fused into the gate/up matmul: both in the 16-row MFMA layout with the same shape, or a
-// pass of T rows that takes the GEMMs
-bool fused_ffn(const DevMat & g, const DevMat & u, int T) {
+// SwiGLU fused into the gate/up matmul: both in the 16-row MFMA layout with the same shape, or F16 on
+// the GEMM
+bool fused_ffn(const DevMat & g, const DevMat & u) {
     return (g.m16 && u.m16 && g.type == u.type && g.nsb == u.nsb && g.tiles == u.tiles) ||
-           (use_gemm(g, T) && gemm_dual_ok(g, u));
+           (!g.m16 && g.type == Z2H_F16 && gemm_dual_ok(g, u));
 }
 
 int launch_encode(z2h_ctx * ctx, const float * x, int ld, int K, int n_rows, int act_fmt, const ActBuf & act) {
@@ -951,7 +996,7 @@ int expert_block(z2h_ctx * ctx, Layer & ly, int L, int T, const float * state_in
     }
     // routes grouped by expert (mul_mat_id's grouping): the grouped matmul blocks list up to LIST_MAX
     // routes in LDS themselves; larger batches, and captures, take one sort kernel's table
-    const bool sorted = ctx->capture || T * ly.k > LIST_MAX || use_gemm(ly.gate_exps, T) || use_gemm(ly.down_exps, T);
+    const bool sorted = ctx->capture || T * ly.k > LIST_MAX || use_gemm_experts(ly.gate_exps, T, ly.k, ly.E) || use_gemm_experts(ly.down_exps, T, ly.k, ly.E);
     if (sorted) {
         prof_scope ps(ctx, Z2H_KF_ROUTER_TAIL);
         int32_t * cc = ctx->capture ? (int32_t *) capp(ctx, Z2H_CAP_COUNTS, L) : nullptr;
@@ -963,7 +1008,7 @@ int expert_block(z2h_ctx * ctx, Layer & ly, int L, int T, const float * state_in
     if ((rc = cap_copy(ctx, Z2H_CAP_ROUTER_STATE, L, r.rh, T))) return rc;
     if ((rc = cap_copy(ctx, Z2H_CAP_SEL, L, ctx->sel, T))) return rc;
     if ((rc = cap_copy(ctx, Z2H_CAP_WEIGHTS, L, ctx->wsel, T))) return rc;
-    if (fused_ffn(ly.gate_exps, ly.up_exps, T)) {
+    if (fused_ffn(ly.gate_exps, ly.up_exps)) {
         // gate + up + SwiGLU in one grouped launch -> y [route][ff] fp32, encoded once for down
         GemvArgs g{};
         g.grouped = 1; g.n_tok = T; g.sel = ctx->sel; g.k = ly.k; g.act = ctx->act; g.E = ly.E; g.mode = MM_SWIGLU;
@@ -1005,11 +1050,11 @@ int expert_block(z2h_ctx * ctx, Layer & ly, int L, int T, const float * state_in
 int dense_block(z2h_ctx * ctx, Layer & ly, int T) {
     const auto & hp = ctx->hp;
     int rc;
-    if (fused_ffn(ly.ffn_gate, ly.ffn_up, T)) {
+    if (fused_ffn(ly.ffn_gate, ly.ffn_up)) {
         GemvArgs g = gemv_dense(ctx, T, ctx->gu_g, hp.n_ff, EPI_STORE);
         g.mode = MM_SWIGLU;
         if ((rc = launch_gemv(ctx, ly.ffn_gate, &ly.ffn_up, g, 1, Z2H_KF_GEMV_DENSE))) return rc;
-        const bool xf = xf_split_ok(ctx, ly.ffn_down, T, false) && !use_gemm(ly.ffn_down, T);
+        const bool xf = xf_split_ok(ctx, ly.ffn_down, T, false) && !use_gemm(ctx, ly.ffn_down, T);
         if (!xf && (rc = launch_encode(ctx, ctx->gu_g, hp.n_ff, hp.n_ff, T, act_of(ly.ffn_down.type), ctx->act_y))) return rc;
         GemvArgs dn = gemv_dense(ctx, T, ctx->eo, hp.n_embd, EPI_STORE);
         dn.act = ctx->act_y;
@@ -1317,6 +1362,8 @@ int set_lds_limits(std::string & err) {
     LDS_ATTR((k_router_down_t<4, true>)) LDS_ATTR((k_router_down_t<8, true>)) LDS_ATTR((k_router_down_t<16, true>))
     LDS_ATTR((k_router_down_t<32, true>)) LDS_ATTR((k_router_down_t<64, true>))
     LDS_ATTR(k_gemm_q4k<true>) LDS_ATTR(k_gemm_q4k<false>)
+    LDS_ATTR((k_gemm_q80<true, 1>)) LDS_ATTR((k_gemm_q80<true, 2>)) LDS_ATTR((k_gemm_q80<false, 1>)) LDS_ATTR((k_gemm_q80<false, 2>))
+    LDS_ATTR((k_gemm_q6k<true, 1>)) LDS_ATTR((k_gemm_q6k<true, 2>)) LDS_ATTR((k_gemm_q6k<true, 4>)) LDS_ATTR((k_gemm_q6k<false, 1>)) LDS_ATTR((k_gemm_q6k<false, 2>)) LDS_ATTR((k_gemm_q6k<false, 4>))
     LDS_ATTR(k_attn_flash32<1>) LDS_ATTR(k_attn_flash32<2>) LDS_ATTR(k_attn_flash32<4>)
     LDS_ATTR(k_attn_flash16<1>) LDS_ATTR(k_attn_flash16<2>) LDS_ATTR(k_attn_flash16<4>)
     LDS_ATTR((k_gemm_f16<true, 4, 4>)) LDS_ATTR((k_gemm_f16<false, 4, 4>)) LDS_ATTR((k_gemm_f16<true, 2, 1>)) LDS_ATTR((k_gemm_f16<false, 1, 1>))

@@ -100,6 +100,29 @@ __device__ __forceinline__ float gemm_epi(const GemmArgs & a, float y, int it) {
     return y;
 }
 
+// Store a wave's sums: acc[x][ts][i] is token 16 ts + 4 (lane / 16) + i of the block tile by row lane % 16
+// of 16-row group grp[x] (DUAL: x = 0 gate, 1 up, SwiGLU).
+template <bool DUAL, int NG, int TS>
+__device__ __forceinline__ void gemm_store(const GemmArgs & a, const float (&acc)[NG][TS][4], const int (&grp)[NG], int lane,
+                                           int nt, const int * s_out) {
+#pragma unroll
+    for (int ts = 0; ts < TS; ++ts)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = ts * 16 + 4 * (lane >> 4) + i;
+            if (t >= nt) continue;
+            const int it = s_out[t];
+            float * o = a.out + (int64_t) it * a.out_ld;
+#pragma unroll
+            for (int x = 0; x < (DUAL ? 1 : NG); ++x) {
+                const int row = grp[x] * 16 + (lane & 15);
+                if (grp[x] >= a.tiles || row >= a.rows) continue;
+                if constexpr (DUAL) o[row] = acc[1][ts][i] * z_silu(acc[0][ts][i]);
+                else o[row] = gemm_epi(a, acc[x][ts][i], it);
+            }
+        }
+}
+
 // ------------------------------------------------------------------ Q4_K x Q8_K
 // One superblock of GM_T activation rows in registers (GM_T / 16 x 16 B of values, GM_T / 32 sub-block
 // sum pairs and the block scale per thread), then in LDS: values [GM_T][GM_QP], sums as f16 pairs
