@@ -911,6 +911,53 @@ RouterArgs router_args(z2h_ctx * ctx, const Layer & ly, int L, int T, const floa
 // router-down elements per lane: the next power of two >= ceil(d / 64); unguarded when d fills every lane
 int router_ni(int d) { return d <= 64 ? 1 : 1 << (32 - __builtin_clz((unsigned) ((d + 63) / 64 - 1))); }
 
+// Wide passes take the router down projection that reuses each weight row across RD_T tokens
+// (k_router_down_t); same bits per token as the per-token kernels.
+bool router_down_wide(const z2h_ctx * ctx, int T) {
+    return T >= GEMM_MIN_ROWS && router_ni(ctx->hp.n_embd) % 4 == 0 && ctx->rd % 32 == 0;
+}
+
+int launch_router_down_t(z2h_ctx * ctx, const RouterArgs & r) {
+    const int ni = router_ni(ctx->hp.n_embd);
+    const dim3 grid(ctx->rd / 32, (r.T + RD_T - 1) / RD_T);
+    const size_t lds = router_down_t_lds(ni);
+#define RDT(N_) do { if (ctx->hp.n_embd == 64 * ni) KL((k_router_down_t<N_, false>), grid, dim3(256), lds, ctx->stream, r); \
+                     else KL((k_router_down_t<N_, true>), grid, dim3(256), lds, ctx->stream, r); } while (0)
+    switch (ni) {
+        case 4: RDT(4); break;
+        case 8: RDT(8); break;
+        case 16: RDT(16); break;
+        case 32: RDT(32); break;
+        default: RDT(64); break;
+    }
+#undef RDT
+    HIPX(hipGetLastError());
+    return Z2H_OK;
+}
+
+// the router down projection alone (k_ffn_entry has it fused with the norm)
+int launch_router_down(z2h_ctx * ctx, const RouterArgs & r) {
+    prof_scope ps(ctx, Z2H_KF_ROUTER_DOWN);
+    if (router_down_wide(ctx, r.T)) return launch_router_down_t(ctx, r);
+    const dim3 grid((ctx->rd + 3) / 4, r.T);
+    const int ni = router_ni(ctx->hp.n_embd);
+    const bool exact = ctx->hp.n_embd == 64 * ni;
+#define RDN(N_) do { if (exact) KL((k_router_down<N_, false>), grid, dim3(256), 0, ctx->stream, r); \
+                     else KL((k_router_down<N_, true>), grid, dim3(256), 0, ctx->stream, r); } while (0)
+    switch (ni) {
+        case 1: RDN(1); break;
+        case 2: RDN(2); break;
+        case 4: RDN(4); break;
+        case 8: RDN(8); break;
+        case 16: RDN(16); break;
+        case 32: RDN(32); break;
+        default: RDN(64); break;
+    }
+#undef RDN
+    HIPX(hipGetLastError());
+    return Z2H_OK;
+}
+
 // An MoE layer's FFN entry as one launch (k_ffn_entry): res_out = res_in + src, x = ffn_norm(res_out)
 // into ctx->cur and the expert activations, router-down state of layer L.
 int launch_ffn_entry(z2h_ctx * ctx, const Layer & ly, int L, int T, const float * state_in,
@@ -923,25 +970,12 @@ int launch_ffn_entry(z2h_ctx * ctx, const Layer & ly, int L, int T, const float 
     f.eps = hp.rms_eps; f.cur_out = ctx->cur; f.act = ctx->act; f.act_fmt = act_of(ly.up_exps.type); f.err = ctx->d_err;
     const int ni = router_ni(hp.n_embd);
     const bool exact = hp.n_embd == 64 * ni;
-    if (T >= GEMM_MIN_ROWS && ni % 4 == 0 && ctx->rd % 32 == 0) {
+    if (router_down_wide(ctx, T)) {
         // wide passes: the norm once per token (k_resnorm, the same arithmetic), then the router down
         // projection with each weight row reused across RD_T tokens
         f.res = res_out; f.res_in = res_in;
         if (int rc = launch_resnorm(ctx, T, f)) return rc;
-        const dim3 g2(ctx->rd / 32, (T + RD_T - 1) / RD_T);
-        const size_t l2 = router_down_t_lds(ni);
-#define RDT(N_) do { if (exact) KL((k_router_down_t<N_, false>), g2, dim3(256), l2, ctx->stream, r); \
-                     else KL((k_router_down_t<N_, true>), g2, dim3(256), l2, ctx->stream, r); } while (0)
-        switch (ni) {
-            case 4: RDT(4); break;
-            case 8: RDT(8); break;
-            case 16: RDT(16); break;
-            case 32: RDT(32); break;
-            default: RDT(64); break;
-        }
-#undef RDT
-        HIPX(hipGetLastError());
-        return Z2H_OK;
+        return launch_router_down_t(ctx, r);
     }
     const dim3 grid((ctx->rd + 3) / 4, T);
     const size_t lds = (size_t) kpad(hp.n_embd) * 4;
@@ -967,25 +1001,7 @@ int expert_block(z2h_ctx * ctx, Layer & ly, int L, int T, const float * state_in
     int rc;
     // router (exact contract)
     const RouterArgs r = router_args(ctx, ly, L, T, state_in);
-    if (!down_done) {
-        prof_scope ps(ctx, Z2H_KF_ROUTER_DOWN);
-        const dim3 grid((ctx->rd + 3) / 4, T);
-        const int ni = router_ni(hp.n_embd);
-        const bool exact = hp.n_embd == 64 * ni;
-#define RDN(N_) do { if (exact) KL((k_router_down<N_, false>), grid, dim3(256), 0, ctx->stream, r); \
-                     else KL((k_router_down<N_, true>), grid, dim3(256), 0, ctx->stream, r); } while (0)
-        switch (ni) {
-            case 1: RDN(1); break;
-            case 2: RDN(2); break;
-            case 4: RDN(4); break;
-            case 8: RDN(8); break;
-            case 16: RDN(16); break;
-            case 32: RDN(32); break;
-            default: RDN(64); break;
-        }
-#undef RDN
-        HIPX(hipGetLastError());
-    }
+    if (!down_done && (rc = launch_router_down(ctx, r))) return rc;
     {
         prof_scope ps(ctx, Z2H_KF_ROUTER_TAIL);
         // wide passes: up to one block per compute unit, each looping over its tokens with the MLP
