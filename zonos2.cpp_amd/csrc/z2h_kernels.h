@@ -394,10 +394,9 @@ __global__ void __launch_bounds__(256) k_resnorm(ResNormArgs a) {
             bool bad = false;
 #pragma unroll
             for (int kk = 0; kk < TW; ++kk) {
-                const int kc = min(kk, a.W - 1);
-                const bool ok = ids[kk] >= 0 && ids[kk] < a.tab_rows[kc];
-                bad = bad || !ok;
-                rows[kk] = a.tab[kc] + (int64_t) (ok ? ids[kk] : 0) * rb;
+                const bool in = kk < a.W, ok = ids[kk] >= 0 && ids[kk] < a.tab_rows[kk];
+                bad = bad || (in && !ok);
+                rows[kk] = in ? a.tab[kk] + (int64_t) (ok ? ids[kk] : 0) * rb : rows[0];
             }
             if (bad && tid == 0) atomicOr(a.err, 1);
 #pragma unroll
@@ -411,8 +410,11 @@ __global__ void __launch_bounds__(256) k_resnorm(ResNormArgs a) {
                 float4 x = e[0];
 #pragma unroll
                 for (int kk = 1; kk < TW; ++kk) {
+                    // (by component: choosing between two float4 objects puts them in scratch memory: the
+                    // kernel took 73 us for 2088 rows of 10 tables x 2048 that way, 23 us this way)
                     const float4 y = add4(x, e[kk]);
-                    x = kk < a.W ? y : x;
+                    const bool in = kk < a.W;
+                    x = make_float4(in ? y.x : x.x, in ? y.y : x.y, in ? y.z : x.z, in ? y.w : x.w);
                 }
                 xv[j] = x;
             }
