@@ -35,9 +35,7 @@ extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, false, true>(
 extern template __global__ void k_gemv_split<WF_Q8_0, true, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, true, true>(GemvArgs);
-// the quantized GEMMs, instantiated in z2h_wide.hip
-extern template __global__ void k_gemm_q4k<true>(GemmArgs);
-extern template __global__ void k_gemm_q4k<false>(GemmArgs);
+// the Q8_0 and Q6_K GEMMs, instantiated in z2h_wide.hip
 extern template __global__ void k_gemm_q80<true, 1>(GemmArgs);
 extern template __global__ void k_gemm_q80<true, 2>(GemmArgs);
 extern template __global__ void k_gemm_q80<false, 1>(GemmArgs);
@@ -629,16 +627,14 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 //                top-4 of 32: Q6_K gate/up 38 us against 52, down 22 against 32; 48 rows, 6 routes: level
 //                before the sort launch is counted).
 constexpr int GEMM_MIN_ROWS = 65;
-// (k_gemm_q4k's activation offsets are 32-bit)
-bool gemm_q4k_ok(const DevMat & m, int64_t items) { return items * m.nsb * 256 < (int64_t) 1 << 32; }
 bool use_gemm(const z2h_ctx * ctx, const DevMat & m, int n_tok) {
     if (!m.m16) return m.type == Z2H_F16;
-    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, n_tok);
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
     return n_tok > 2 && 2ll * ((m.tiles + 3) / 4) * ((n_tok + 15) / 16) > ctx->n_cu;
 }
 bool use_gemm_experts(const DevMat & m, int n_tok, int k, int E) {
     if (!m.m16) return m.type == Z2H_F16;
-    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, (int64_t) n_tok * k);
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
     return n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
 }
 // gate and up fused with SwiGLU in one GEMM launch: same type, layout and shape
@@ -665,9 +661,9 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
     a.r_off = g.r_off; a.r_perm = g.r_perm; a.act = g.act;
     a.out = g.out[0]; a.out_ld = g.out_ld; a.epi = g.epi; a.cap = g.cap; a.route_w = g.route_w;
     if (m0.type == Z2H_Q4_K) {
-        const dim3 grid(dual ? (m0.tiles + 3) / 4 : (m0.tiles + 7) / 8, gemm_slots(a.grouped, a.n_tok, a.k, a.E, Q4_T));
-        if (dual) KL(k_gemm_q4k<true>, grid, dim3(256), gemm_q4k_lds, ctx->stream, a);
-        else KL(k_gemm_q4k<false>, grid, dim3(256), gemm_q4k_lds, ctx->stream, a);
+        const dim3 grid(dual ? (m0.tiles + 3) / 4 : (m0.tiles + 7) / 8, gemm_slots(a.grouped, a.n_tok, a.k, a.E, GM_T));
+        if (dual) KL(k_gemm_q4k<true>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
+        else KL(k_gemm_q4k<false>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
     } else if (m0.m16) {
         // the tallest token tile that is half full on average and leaves at least two blocks per compute
         // unit (grouped launches fill about routes / GT + E / 2 tile slots): 333 rows of Q8_0 W_o 11.0 us
@@ -915,7 +911,7 @@ RouterArgs router_args(z2h_ctx * ctx, const Layer & ly, int L, int T, const floa
 // router-down elements per lane: the next power of two >= ceil(d / 64); unguarded when d fills every lane
 int router_ni(int d) { return d <= 64 ? 1 : 1 << (32 - __builtin_clz((unsigned) ((d + 63) / 64 - 1))); }
 
-// Wide passes take the router down projection that reuses each weight row across a block's tokens
+// Wide passes take the router down projection that reuses each weight row across RD_T tokens
 // (k_router_down_t); same bits per token as the per-token kernels.
 bool router_down_wide(const z2h_ctx * ctx, int T) {
     return T >= GEMM_MIN_ROWS && router_ni(ctx->hp.n_embd) % 4 == 0 && ctx->rd % 32 == 0;
@@ -923,12 +919,9 @@ bool router_down_wide(const z2h_ctx * ctx, int T) {
 
 int launch_router_down_t(z2h_ctx * ctx, const RouterArgs & r) {
     const int ni = router_ni(ctx->hp.n_embd);
-    // two blocks per compute unit (registers)
-    const int gx = ctx->rd / 16;
-    const dim3 grid(gx, std::min((r.T + RD_T - 1) / RD_T, std::max(1, 2 * ctx->n_cu / gx)));
-    const size_t lds = router_down_t_lds(ni, ctx->hp.n_embd);
-    const bool exact = ctx->hp.n_embd == 64 * ni;
-#define RDT(N_) do { if (exact) KL((k_router_down_t<N_, false>), grid, dim3(256), lds, ctx->stream, r); \
+    const dim3 grid(ctx->rd / 32, (r.T + RD_T - 1) / RD_T);
+    const size_t lds = router_down_t_lds(ni);
+#define RDT(N_) do { if (ctx->hp.n_embd == 64 * ni) KL((k_router_down_t<N_, false>), grid, dim3(256), lds, ctx->stream, r); \
                      else KL((k_router_down_t<N_, true>), grid, dim3(256), lds, ctx->stream, r); } while (0)
     switch (ni) {
         case 4: RDT(4); break;
@@ -979,7 +972,7 @@ int launch_ffn_entry(z2h_ctx * ctx, const Layer & ly, int L, int T, const float 
     const bool exact = hp.n_embd == 64 * ni;
     if (router_down_wide(ctx, T)) {
         // wide passes: the norm once per token (k_resnorm, the same arithmetic), then the router down
-        // projection with each weight row reused across a block's tokens
+        // projection with each weight row reused across RD_T tokens
         f.res = res_out; f.res_in = res_in;
         if (int rc = launch_resnorm(ctx, T, f)) return rc;
         return launch_router_down_t(ctx, r);
@@ -1380,9 +1373,10 @@ int set_lds_limits(std::string & err) {
     LDS_ATTR((k_gemv_mfma<WF_Q6_K, false, MT, 1>)) LDS_ATTR((k_gemv_mfma<WF_Q6_K, true, MT, 1>))
     LDS_ATTR((k_gemv_split<WF_Q6_K, false, MT>)) LDS_ATTR((k_gemv_split<WF_Q6_K, true, MT>))
     LDS_ATTR((k_gemv_split<WF_Q6_K, false, MT_G>)) LDS_ATTR((k_gemv_split<WF_Q6_K, true, MT_G>))
-#define LDS_RDT(N_) LDS_ATTR((k_router_down_t<N_, false>)) LDS_ATTR((k_router_down_t<N_, true>))
-    LDS_RDT(4) LDS_RDT(8) LDS_RDT(16) LDS_RDT(32) LDS_RDT(64)
-#undef LDS_RDT
+    LDS_ATTR((k_router_down_t<4, false>)) LDS_ATTR((k_router_down_t<8, false>)) LDS_ATTR((k_router_down_t<16, false>))
+    LDS_ATTR((k_router_down_t<32, false>)) LDS_ATTR((k_router_down_t<64, false>))
+    LDS_ATTR((k_router_down_t<4, true>)) LDS_ATTR((k_router_down_t<8, true>)) LDS_ATTR((k_router_down_t<16, true>))
+    LDS_ATTR((k_router_down_t<32, true>)) LDS_ATTR((k_router_down_t<64, true>))
     LDS_ATTR(k_gemm_q4k<true>) LDS_ATTR(k_gemm_q4k<false>)
     LDS_ATTR((k_gemm_q80<true, 1>)) LDS_ATTR((k_gemm_q80<true, 2>)) LDS_ATTR((k_gemm_q80<false, 1>)) LDS_ATTR((k_gemm_q80<false, 2>))
     LDS_ATTR((k_gemm_q6k<true, 1>)) LDS_ATTR((k_gemm_q6k<true, 2>)) LDS_ATTR((k_gemm_q6k<true, 4>)) LDS_ATTR((k_gemm_q6k<false, 1>)) LDS_ATTR((k_gemm_q6k<false, 2>)) LDS_ATTR((k_gemm_q6k<false, 4>))
@@ -2305,7 +2299,7 @@ static int sample_impl(z2h_ctx * ctx, int n_active, const float * d_logits, cons
     if (hist && (hist_cap < 0 || hist_cap > Z2H_SAMPLE_HIST_MAX || !hist_len))
         return seterr(ctx, Z2H_EINVAL, "history capacity out of range (at most Z2H_SAMPLE_HIST_MAX)");
     const int ncb = ctx->hp.n_codebooks, av = ctx->hp.audio_vocab;
-    int np2 = 256;
+    int np2 = 1;
     while (np2 < av) np2 <<= 1;
     if (ncb <= 0 || av <= 0 || np2 > 4096) return seterr(ctx, Z2H_ENOTSUP, "audio vocabulary too large for the sampler");
     const int hc = hist ? hist_cap : 0;
