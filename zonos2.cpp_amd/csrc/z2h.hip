@@ -2299,7 +2299,7 @@ static int sample_impl(z2h_ctx * ctx, int n_active, const float * d_logits, cons
     if (hist && (hist_cap < 0 || hist_cap > Z2H_SAMPLE_HIST_MAX || !hist_len))
         return seterr(ctx, Z2H_EINVAL, "history capacity out of range (at most Z2H_SAMPLE_HIST_MAX)");
     const int ncb = ctx->hp.n_codebooks, av = ctx->hp.audio_vocab;
-    int np2 = 1;
+    int np2 = 256;
     while (np2 < av) np2 <<= 1;
     if (ncb <= 0 || av <= 0 || np2 > 4096) return seterr(ctx, Z2H_ENOTSUP, "audio vocabulary too large for the sampler");
     const int hc = hist ? hist_cap : 0;

@@ -2913,7 +2913,7 @@ __global__ void __launch_bounds__(RT_THREADS) k_router_tail(RouterArgs a) {
 struct SampleParams { float temperature; int top_k; float top_p; float min_p; float rep_penalty; int rep_codebooks; int greedy; int pad; };
 struct SampleArgs {
     const float * logits;             // [n][ncb][av]
-    int ncb, av, np2;                 // np2 = power of two >= av (sort width)
+    int ncb, av, np2;                 // np2 = power of two >= av and >= 256 (sort width)
     const SampleParams * sp;          // [n]
     const int32_t * hist; const int32_t * hlen; int hcap;   // [n][ncb][hcap] codes, [n][ncb] counts
     const double * u;                 // [n][ncb] canonical draws in [0, 1)
@@ -2927,14 +2927,141 @@ __host__ __device__ inline size_t sample_lds_bytes(int av, int np2) { return (si
 // id order), p = exp(l - max) over a double sum, top-p along the probability order, min-p against the
 // largest p, and the draw r = u * mass walked along the candidates (no draw is used where the kept
 // mass is 0: the code is then the first id of the probability order). The ranking is a bitonic sort
-// of (logit descending, id ascending) over np2 entries in LDS; the order-dependent sums (normaliser,
-// kept mass, the walk) run in one thread in candidate order, as the reference's loops do. Where equal
+// of (logit descending, id ascending) over np2 entries in registers (sample_sort). The order-dependent sums
+// (normaliser, kept mass, the walk) keep the reference's candidate order: one wave holds 64 terms in its lanes
+// and adds them one by one (sample_seq). A history's occurrences of one id are applied to that id in a row, which is
+// the reference's result: each touches its own id only. Where equal
 // logits or probabilities could change the code, the decisions run again on the exact orders of
 // std::partial_sort / std::sort (z2h_order), so the codes are the reference's with ties too.
+// Bounded by these chains' latency (one block per draw, few per compute unit). 16 columns x 9 codebooks x
+// 1026 ids, histories of 64, top-k 100: 88 us with the penalties, sums and decisions in one thread and the sort's
+// 66 stages through LDS; 26 us.
+
+// lane l's partner l ^ M of a value (M = 1 .. 32), by DPP and lane swaps
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor_u(uint32_t v, int lane) {
+    const int i = (int) v;
+    if constexpr (M == 1) return (uint32_t) dpp_i<DPP_QUAD_XOR1>(i);
+    else if constexpr (M == 2) return (uint32_t) dpp_i<DPP_QUAD_XOR2>(i);
+    else if constexpr (M == 4) return (uint32_t) dpp_i<0x1B>(dpp_i<DPP_ROW_HALF_MIRROR>(i));   // (7 - l, then quads reversed)
+    else if constexpr (M == 8) return (uint32_t) dpp_i<0x128>(i);                              // row rotated by 8
+    else if constexpr (M == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (lane & 16) ? r[0] : r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (lane & 32) ? r[0] : r[1];
+    }
+}
+
+// Bitonic sort of 256 E keys, descending, by a 256-thread block: thread tid holds positions E tid .. E tid +
+// E - 1 in x. Strides below E stay in the thread, below 64 E in the wave (lane swaps), the last two go
+// through buf[256 E]. One stage per call; the strides are compile-time so that x stays in registers.
+template <int E, int STRIDE>
+__device__ __forceinline__ void sample_stage(uint64_t (&x)[E], int size, uint64_t * buf, int tid) {
+    if constexpr (STRIDE < E) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            if (i & STRIDE) continue;
+            const bool desc = ((E * tid + i) & size) == 0;
+            const uint64_t l = x[i], h = x[i + STRIDE];
+            const bool sw = (h > l) == desc;
+            x[i] = sw ? h : l;
+            x[i + STRIDE] = sw ? l : h;
+        }
+    } else {
+        constexpr int M = STRIDE / E;                                // partner thread tid ^ M
+        if constexpr (M >= 64) {
+            __syncthreads();                                         // earlier reads of buf are done
+#pragma unroll
+            for (int i = 0; i < E; ++i) buf[256 * i + tid] = x[i];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            uint64_t o;
+            if constexpr (M >= 64) o = buf[256 * i + (tid ^ M)];
+            else o = ((uint64_t) lane_xor_u<(M < 64 ? M : 1)>((uint32_t) (x[i] >> 32), tid & 63) << 32) |
+                     lane_xor_u<(M < 64 ? M : 1)>((uint32_t) x[i], tid & 63);
+            // the lower position of the pair keeps the larger key where the run descends
+            const bool big = (((E * tid + i) & size) == 0) == ((tid & M) == 0);
+            x[i] = (o > x[i]) == big ? o : x[i];
+        }
+    }
+}
+template <int E, int STRIDE>
+__device__ __forceinline__ void sample_merge(uint64_t (&x)[E], int size, uint64_t * buf, int tid) {
+    sample_stage<E, STRIDE>(x, size, buf, tid);
+    if constexpr (STRIDE > 1) sample_merge<E, STRIDE / 2>(x, size, buf, tid);
+}
+template <int E, int SIZE>
+__device__ __forceinline__ void sample_sort_from(uint64_t (&x)[E], uint64_t * buf, int tid) {
+    sample_merge<E, SIZE / 2>(x, SIZE, buf, tid);
+    if constexpr (SIZE < 256 * E) sample_sort_from<E, SIZE * 2>(x, buf, tid);
+}
+
+// The ids 0 .. av - 1 by s_lg descending, equal logits by id ascending, then pads: ranks' logits to s_key, ids
+// to s_idx (np2 = 256 E entries, adjacent: together the exchange buffer). Key: the logit's bits made
+// order-preserving (-0 as +0: they compare equal; a NaN as -inf, so that ids stay ahead of pads), then ~id.
+template <int E>
+__device__ __forceinline__ void sample_sort(const float * s_lg, int av, float * s_key, int * s_idx) {
+    const int tid = threadIdx.x;
+    uint64_t * buf = (uint64_t *) s_key;
+    uint64_t x[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int id = tid + 256 * i;                                // (any start order: the keys are distinct)
+        const float v = id < av ? s_lg[id] : -__builtin_inff();
+        const uint32_t b = __builtin_bit_cast(uint32_t, v == v ? v + 0.0f : -__builtin_inff());
+        const uint32_t m = b ^ ((uint32_t) ((int32_t) b >> 31) | 0x80000000u);
+        x[i] = ((uint64_t) m << 32) | (uint32_t) ~id;
+    }
+    sample_sort_from<E, 2>(x, buf, tid);
+    __syncthreads();                                                 // the last exchange is read
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int id = (int) ~(uint32_t) x[i];
+        s_idx[E * tid + i] = id;
+        s_key[E * tid + i] = id < av ? s_lg[id] : -__builtin_inff();
+    }
+}
+
+// The running sum of val(0), val(1), ..., val(n - 1) in that order, in double, by one wave: returns the first j whose
+// sum reaches `target` (n if none), total = the sum of all terms where none does. (Terms past n add 0.)
+template <bool FIND, class Val>
+__device__ __forceinline__ int sample_seq(int n, Val val, double target, double & total) {
+    const int lane = threadIdx.x & 63;
+    double acc = 0.0;
+    for (int c0 = 0; c0 < n; c0 += 64) {
+        const int j = c0 + lane;
+        const float v = j < n ? val(j) : 0.0f;
+        double mine = 0.0;
+        for (int l0 = 0; l0 < min(64, n - c0); l0 += 16) {
+#pragma unroll
+            for (int l = 0; l < 16; ++l) {
+                acc = acc + (double) __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l0 + l));
+                if (FIND) mine = lane == l0 + l ? acc : mine;
+            }
+        }
+        if (FIND) {
+            const uint64_t hit = __ballot(j < n && mine >= target);
+            if (hit) { total = acc; return c0 + (int) __ffsll((unsigned long long) hit) - 1; }
+        }
+    }
+    total = acc;
+    return n;
+}
+// LDS writes of one lane before the wave's reads
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 #ifndef Z2H_TEMPLATES_ONLY
 __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
     extern __shared__ __attribute__((aligned(16))) char sm_s[];
-    float * s_key = (float *) sm_s;                              // [np2]
+    float * s_key = (float *) sm_s;                              // [np2] (with s_idx, the sort's exchange buffer first)
     int * s_idx = (int *) (s_key + a.np2);                       // [np2]
     float * s_lg = (float *) (s_idx + a.np2);                    // [av] penalised / tempered logits by id
     float * s_p = s_lg + a.av;                                   // [av] probabilities by candidate
@@ -2960,39 +3087,34 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
         }
         return;
     }
-    for (int j = tid; j < av; j += 256) s_lg[j] = in[j];
-    __syncthreads();
-    if (tid == 0 && sp.rep_penalty != 1.0f && cb < sp.rep_codebooks) {
+    // how often each id occurs in the history (s_idx, free before the sort)
+    const bool pen = sp.rep_penalty != 1.0f && cb < sp.rep_codebooks;
+    if (pen) {
+        for (int j = tid; j < av; j += 256) s_idx[j] = 0;
+        __syncthreads();
         const int32_t * h = a.hist + ((size_t) col * a.ncb + cb) * a.hcap;
-        const int n = min(a.hlen[(size_t) col * a.ncb + cb], a.hcap);
-        for (int i = 0; i < n; ++i) {
+        const int nh = min(a.hlen[(size_t) col * a.ncb + cb], a.hcap);
+        for (int i = tid; i < nh; i += 256) {
             const int t = h[i];
-            if (t >= 0 && t < av) s_lg[t] = s_lg[t] > 0.0f ? s_lg[t] / sp.rep_penalty : s_lg[t] * sp.rep_penalty;
+            if (t >= 0 && t < av) atomicAdd(&s_idx[t], 1);
         }
+        __syncthreads();
+    }
+    for (int j = tid; j < av; j += 256) {
+        float v = in[j];
+        if (pen) for (int c = s_idx[j]; c > 0; --c) v = v > 0.0f ? v / sp.rep_penalty : v * sp.rep_penalty;
+        if (sp.temperature > 0.0f) v = v / sp.temperature;
+        s_lg[j] = v;
     }
     __syncthreads();
-    for (int j = tid; j < np2; j += 256) {
-        float v = -__builtin_inff();
-        if (j < av) {
-            v = s_lg[j];
-            if (sp.temperature > 0.0f) { v = v / sp.temperature; s_lg[j] = v; }
-        }
-        s_key[j] = v; s_idx[j] = j;
+    switch (np2) {
+        case 256: sample_sort<1>(s_lg, av, s_key, s_idx); break;
+        case 512: sample_sort<2>(s_lg, av, s_key, s_idx); break;
+        case 1024: sample_sort<4>(s_lg, av, s_key, s_idx); break;
+        case 2048: sample_sort<8>(s_lg, av, s_key, s_idx); break;
+        default: sample_sort<16>(s_lg, av, s_key, s_idx); break;
     }
     __syncthreads();
-    // bitonic sort, descending by logit, ties to the lower id
-    for (int size = 2; size <= np2; size <<= 1)
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = tid; i < np2 / 2; i += 256) {
-                const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
-                const float kl = s_key[lo], kh = s_key[hi];
-                const int il = s_idx[lo], ih = s_idx[hi];
-                const bool hi_first = kh > kl || (kh == kl && ih < il);
-                const bool desc = (lo & size) == 0;
-                if (desc ? hi_first : !hi_first) { s_key[lo] = kh; s_key[hi] = kl; s_idx[lo] = ih; s_idx[hi] = il; }
-            }
-            __syncthreads();
-        }
     const bool topk = sp.top_k > 0 && sp.top_k < av;
     const int n = topk ? sp.top_k : av;
     // candidate j: id s_idx[j] (top-k) or j (all ids); probability-rank r: candidate r (top-k: the
@@ -3002,12 +3124,16 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
     for (int j = tid; j < n; j += 256) { s_p[j] = z_expf_cr(s_lg[cand(j)] - mx); s_keep[j] = 1; }
     __syncthreads();
     __shared__ double s_z;
-    if (tid == 0) { double z = 0.0; for (int j = 0; j < n; ++j) z += (double) s_p[j]; s_z = z; }
+    if (wave == 0) {
+        double z;
+        sample_seq<false>(n, [&](int j) { return s_p[j]; }, 0.0, z);
+        if (lane == 0) s_z = z;
+    }
     __syncthreads();
     const double z = s_z;
     for (int j = tid; j < n; j += 256) s_p[j] = (float) ((double) s_p[j] / z);
     __syncthreads();
-    if (tid != 0) return;
+    if (wave != 0) return;
     // The decisions run along two orders: the candidate order (the walk) and the probability order
     // (top-p, the min-p reference, the fallback). Where keys are distinct, the bitonic orders are the
     // reference's. Where equal keys make the reference's order depend on std::partial_sort /
@@ -3015,42 +3141,35 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
     // can hold another id. So the first pass flags the cases where an equal-key neighbour could swap
     // the outcome: a top-p cut inside a run of equal probabilities, a fallback whose top probability
     // is shared, or a code whose logit is shared (top-k). Those cases run again on the library's
-    // exact orders (z2h_order, one thread).
+    // exact orders (z2h_order, one thread). The wave's lanes decide together; every lane has the answer.
     const double top_p = sp.top_p > 0.0f && sp.top_p < 1.0f ? (double) sp.top_p : -1.0;
     auto decide = [&](auto cand_at, auto rank_at, bool flag_ties, bool & tie) -> int {
         tie = false;
+        double total;
         if (top_p > 0.0) {
-            double c = 0.0; bool reached = false;
-            for (int r = 0; r < n; ++r) {
-                const int j = rank_at(r);
-                if (reached) s_keep[j] = 0;
-                c += (double) s_p[j];
-                if (!reached && c >= top_p) {
-                    reached = true;
-                    if (flag_ties && r + 1 < n && s_p[rank_at(r + 1)] == s_p[j]) tie = true;
-                }
-            }
+            const int r = sample_seq<true>(n, [&](int q) { return s_p[rank_at(q)]; }, top_p, total);
+            if (flag_ties && r + 1 < n && s_p[rank_at(r + 1)] == s_p[rank_at(r)]) tie = true;
+            for (int q = r + 1 + lane; q < n; q += 64) s_keep[rank_at(q)] = 0;
         }
         const int j0 = rank_at(0);
         if (sp.min_p > 0.0f) {
             const float floor_p = sp.min_p * s_p[j0];
-            for (int j = 0; j < n; ++j) if (s_p[j] < floor_p) s_keep[j] = 0;
+            for (int j = lane; j < n; j += 64) if (s_p[j] < floor_p) s_keep[j] = 0;
         }
-        double mass = 0.0;
-        for (int j = 0; j < n; ++j) mass += s_keep[j] ? (double) s_p[j] : 0.0;
+        wave_lds_sync();
+        auto kept = [&](int j) { return s_keep[j] ? s_p[j] : 0.0f; };
+        double mass;
+        sample_seq<false>(n, kept, 0.0, mass);
         // equal logits around candidate position j (top-k: the candidate order is the logit order)
         auto shared_logit = [&](int j) {
             return topk && ((j > 0 && s_key[j - 1] == s_key[j]) || (j + 1 < av && s_key[j + 1] == s_key[j]));
         };
         if (mass > 0.0) {
             const double r = a.u[(size_t) col * a.ncb + cb] * (mass - 0.0) + 0.0;
-            double acc = 0.0;
-            for (int j = 0; j < n; ++j) {
-                acc += s_keep[j] ? (double) s_p[j] : 0.0;
-                if (acc >= r) {
-                    if (flag_ties && shared_logit(j)) tie = true;
-                    return cand_at(j);
-                }
+            const int j = sample_seq<true>(n, kept, r, total);
+            if (j < n) {
+                if (flag_ties && shared_logit(j)) tie = true;
+                return cand_at(j);
             }
         }
         if (flag_ties && ((n > 1 && s_p[rank_at(1)] == s_p[j0]) || shared_logit(j0))) tie = true;
@@ -3062,16 +3181,20 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
         // the library's orders: ids by logit (std::partial_sort over all ids, first top_k kept), then
         // candidate positions by probability (std::sort); s_key is free now and holds the id arrays
         int * ord = (int *) s_key;
-        if (topk) {
-            for (int i = 0; i < av; ++i) ord[i] = i;
-            z2h_order::partial_order(ord, n, av, [&](int x, int y) { return s_lg[x] > s_lg[y]; });
-            for (int j = 0; j < n; ++j) s_idx[j] = ord[j];
+        wave_lds_sync();
+        if (lane == 0) {
+            if (topk) {
+                for (int i = 0; i < av; ++i) ord[i] = i;
+                z2h_order::partial_order(ord, n, av, [&](int x, int y) { return s_lg[x] > s_lg[y]; });
+                for (int j = 0; j < n; ++j) s_idx[j] = ord[j];
+            }
+            for (int j = 0; j < n; ++j) { ord[j] = j; s_keep[j] = 1; }
+            z2h_order::sort_order(ord, n, [&](int x, int y) { return s_p[x] > s_p[y]; });
         }
-        for (int j = 0; j < n; ++j) { ord[j] = j; s_keep[j] = 1; }
-        z2h_order::sort_order(ord, n, [&](int x, int y) { return s_p[x] > s_p[y]; });
+        wave_lds_sync();
         code = decide([&](int j) { return topk ? s_idx[j] : j; }, [&](int r) { return ord[r]; }, false, tie);
     }
-    *out = code;
+    if (lane == 0) *out = code;
 }
 #endif
 
