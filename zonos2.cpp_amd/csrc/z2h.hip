@@ -911,7 +911,7 @@ RouterArgs router_args(z2h_ctx * ctx, const Layer & ly, int L, int T, const floa
 // router-down elements per lane: the next power of two >= ceil(d / 64); unguarded when d fills every lane
 int router_ni(int d) { return d <= 64 ? 1 : 1 << (32 - __builtin_clz((unsigned) ((d + 63) / 64 - 1))); }
 
-// Wide passes take the router down projection that reuses each weight row across RD_T tokens
+// Wide passes take the router down projection that reuses each weight row across a block's tokens
 // (k_router_down_t); same bits per token as the per-token kernels.
 bool router_down_wide(const z2h_ctx * ctx, int T) {
     return T >= GEMM_MIN_ROWS && router_ni(ctx->hp.n_embd) % 4 == 0 && ctx->rd % 32 == 0;
@@ -919,9 +919,12 @@ bool router_down_wide(const z2h_ctx * ctx, int T) {
 
 int launch_router_down_t(z2h_ctx * ctx, const RouterArgs & r) {
     const int ni = router_ni(ctx->hp.n_embd);
-    const dim3 grid(ctx->rd / 32, (r.T + RD_T - 1) / RD_T);
-    const size_t lds = router_down_t_lds(ni);
-#define RDT(N_) do { if (ctx->hp.n_embd == 64 * ni) KL((k_router_down_t<N_, false>), grid, dim3(256), lds, ctx->stream, r); \
+    // two blocks per compute unit (registers)
+    const int gx = ctx->rd / 16;
+    const dim3 grid(gx, std::min((r.T + RD_T - 1) / RD_T, std::max(1, 2 * ctx->n_cu / gx)));
+    const size_t lds = router_down_t_lds(ni, ctx->hp.n_embd);
+    const bool exact = ctx->hp.n_embd == 64 * ni;
+#define RDT(N_) do { if (exact) KL((k_router_down_t<N_, false>), grid, dim3(256), lds, ctx->stream, r); \
                      else KL((k_router_down_t<N_, true>), grid, dim3(256), lds, ctx->stream, r); } while (0)
     switch (ni) {
         case 4: RDT(4); break;
@@ -972,7 +975,7 @@ int launch_ffn_entry(z2h_ctx * ctx, const Layer & ly, int L, int T, const float 
     const bool exact = hp.n_embd == 64 * ni;
     if (router_down_wide(ctx, T)) {
         // wide passes: the norm once per token (k_resnorm, the same arithmetic), then the router down
-        // projection with each weight row reused across RD_T tokens
+        // projection with each weight row reused across a block's tokens
         f.res = res_out; f.res_in = res_in;
         if (int rc = launch_resnorm(ctx, T, f)) return rc;
         return launch_router_down_t(ctx, r);
@@ -1373,10 +1376,9 @@ int set_lds_limits(std::string & err) {
     LDS_ATTR((k_gemv_mfma<WF_Q6_K, false, MT, 1>)) LDS_ATTR((k_gemv_mfma<WF_Q6_K, true, MT, 1>))
     LDS_ATTR((k_gemv_split<WF_Q6_K, false, MT>)) LDS_ATTR((k_gemv_split<WF_Q6_K, true, MT>))
     LDS_ATTR((k_gemv_split<WF_Q6_K, false, MT_G>)) LDS_ATTR((k_gemv_split<WF_Q6_K, true, MT_G>))
-    LDS_ATTR((k_router_down_t<4, false>)) LDS_ATTR((k_router_down_t<8, false>)) LDS_ATTR((k_router_down_t<16, false>))
-    LDS_ATTR((k_router_down_t<32, false>)) LDS_ATTR((k_router_down_t<64, false>))
-    LDS_ATTR((k_router_down_t<4, true>)) LDS_ATTR((k_router_down_t<8, true>)) LDS_ATTR((k_router_down_t<16, true>))
-    LDS_ATTR((k_router_down_t<32, true>)) LDS_ATTR((k_router_down_t<64, true>))
+#define LDS_RDT(N_) LDS_ATTR((k_router_down_t<N_, false>)) LDS_ATTR((k_router_down_t<N_, true>))
+    LDS_RDT(4) LDS_RDT(8) LDS_RDT(16) LDS_RDT(32) LDS_RDT(64)
+#undef LDS_RDT
     LDS_ATTR(k_gemm_q4k<true>) LDS_ATTR(k_gemm_q4k<false>)
     LDS_ATTR((k_gemm_q80<true, 1>)) LDS_ATTR((k_gemm_q80<true, 2>)) LDS_ATTR((k_gemm_q80<false, 1>)) LDS_ATTR((k_gemm_q80<false, 2>))
     LDS_ATTR((k_gemm_q6k<true, 1>)) LDS_ATTR((k_gemm_q6k<true, 2>)) LDS_ATTR((k_gemm_q6k<true, 4>)) LDS_ATTR((k_gemm_q6k<false, 1>)) LDS_ATTR((k_gemm_q6k<false, 2>)) LDS_ATTR((k_gemm_q6k<false, 4>))

@@ -2366,87 +2366,103 @@ __global__ void __launch_bounds__(256) k_router_down(RouterArgs a) {
     if (lane == 0) a.rh[(int64_t) t * a.rd + o] = v;
 }
 
-// k_router_down for wide passes: the same per-(token, output) fma chain, wave tree, bias and state
-// term. A block takes RD_T tokens, whose rows sit in LDS lane-major ([token][lane][j] = x[lane + 64 j],
-// rows padded to NI + 4 floats so the lanes' 16-byte reads fall in distinct banks), and 32 outputs:
-// wave w forms outputs 32 og + 8 w + [0, 8) in groups of OB, each group's weight rows held in
-// registers across the RD_T tokens, so every LDS read of a token's row serves OB independent chains.
-// Grid (rd / 32, ceil(T / RD_T)), 256 threads; tokens past T repeat the last row and are not stored.
-constexpr int RD_T = 8;
-__host__ __device__ inline size_t router_down_t_lds(int ni) { return (size_t) RD_T * 64 * (ni + 4) * 4; }
+// k_router_down for wide passes: the same per-(token, output) fma chains, tree, bias and state term.
+// The 64 chains of an output are spread over 16 lanes, four neighbours per lane (lane p of the group has
+// chains 4p .. 4p + 3: one float4 of the weight row and of the token's row per step), so a wave forms
+// four outputs at once: the tree's first four levels are DPP row shifts inside each 16-lane group, for
+// all four outputs together, and its last two are in the lane; the token's row is one 16-byte LDS read per
+// step that the four groups share. A block keeps its 16 outputs' weights in registers and walks tiles of
+// RD_T tokens, blockIdx.y, blockIdx.y + gridDim.y, ..., the next tile's rows loaded while the present
+// one's chains run; rows of more than 2048 floats go in two halves, the chains kept in LDS between them.
+// Grid (rd / 16, at most ceil(T / RD_T)), 256 threads, dynamic LDS router_down_t_lds(ni, d).
+// Bounded by the LDS return path (each of a token's 16-byte reads serves 4 fma per lane) and by the rows'
+// first load: d 2048, 128 outputs, 77 rows 16.3 -> 6.3 us, 333 16.9 -> 11.5, 1500 41 -> 34, 2088 50 -> 40.
+constexpr int RD_T = 4;
+__host__ __device__ inline size_t router_down_t_lds(int ni, int d) { return (size_t) RD_T * (4 * d + (ni > 32 ? 4096 : 0)); }
 template <int NI, bool GUARD>
-__global__ void __launch_bounds__(256) k_router_down_t(RouterArgs a) {
-    static_assert(NI % 4 == 0, "16-byte LDS reads");
-    constexpr int S = NI + 4, OB = NI >= 64 ? 2 : 4, PER = RD_T * (NI / 4) * 64 / 256;
-    extern __shared__ __attribute__((aligned(16))) float xs_t[];     // [RD_T][64][S]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t0 = blockIdx.y * RD_T;
-    const int nt = min(RD_T, a.T - t0), d = GUARD ? a.d : 64 * NI;
-    // staging item (tt, j4, ln): x[lane ln + 64 (4 j4 + c)], c < 4, as one 16-byte LDS store; every
-    // load is issued before the first store
-    {
-        float4 v[PER];
+__global__ void __launch_bounds__(256, NI > 32 ? 1 : 2) k_router_down_t(RouterArgs a) {
+    constexpr int JH = NI < 32 ? NI : 32, NH = NI / JH, PER = NI / 4;   // PER: float4 per thread of a full tile
+    extern __shared__ __attribute__((aligned(16))) float xs_t[];     // [RD_T][d]
+    const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, d = GUARD ? a.d : 64 * NI;
+    const int o = blockIdx.x * 16 + (tid >> 6) * 4 + (lane >> 4);
+    const float * __restrict__ w = a.w_down + (int64_t) o * d + 4 * p;
+    v4f_t * part = (v4f_t *) (xs_t + (size_t) RD_T * d) + tid;     // (NH > 1) [RD_T][256]: the chains after a half
+    v4f_t wv[JH];
+    auto load_w = [&](int h) {
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int idx = tid + 256 * u, ln = idx & 63, j4 = (idx >> 6) % (NI / 4), tt = (idx >> 6) / (NI / 4);
-            const float * src = a.x + (int64_t) (t0 + min(tt, nt - 1)) * d + ln + 256 * j4;
-            float e[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) e[c] = !GUARD || ln + 64 * (4 * j4 + c) < d ? src[64 * c] : 0.0f;
-            v[u] = make_float4(e[0], e[1], e[2], e[3]);
+        for (int j = 0; j < JH; ++j) {
+            const int i = 64 * (h * JH + j);
+            wv[j] = !GUARD || i + 4 * p < d ? *(const v4f_t *) (w + i) : (v4f_t) {0.0f, 0.0f, 0.0f, 0.0f};
         }
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int idx = tid + 256 * u, ln = idx & 63, j4 = (idx >> 6) % (NI / 4), tt = (idx >> 6) / (NI / 4);
-            *(float4 *) (xs_t + (tt * 64 + ln) * S + 4 * j4) = v[u];
-        }
-    }
-    lds_sync();
+    };
     const bool eda = a.eda && a.state_in;
+    v4f_t x[PER];
+    float st = 0.0f;                                                 // lane p < RD_T: token p's state term
+    const float b = a.b_down[o], se = eda ? a.eda[o] : 0.0f;
+    auto load_x = [&](int t0) {                                      // (items past the tile's rows repeat the last)
+        const int nt = min(RD_T, a.T - t0), n4 = nt * (d / 4);
+        const v4f_t * src = (const v4f_t *) (a.x + (int64_t) t0 * d);
+#pragma unroll
+        for (int u = 0; u < PER; ++u) x[u] = src[min(tid + 256 * u, n4 - 1)];
+        if (eda) st = a.state_in[(int64_t) (t0 + min(p, nt - 1)) * a.rd + o] * se;
+    };
+    load_x(blockIdx.y * RD_T);
+    if (NH == 1) load_w(0);
 #pragma unroll 1
-    for (int g = 0; g < 8 / OB; ++g) {
-        const int o0 = blockIdx.x * 32 + wave * 8 + g * OB;
-        float wv[OB][NI], b[OB];
+    for (int t0 = blockIdx.y * RD_T; t0 < a.T; t0 += gridDim.y * RD_T) {
+        const int nt = min(RD_T, a.T - t0), n4 = RD_T * (d / 4);
 #pragma unroll
-        for (int ob = 0; ob < OB; ++ob) {
-            const float * __restrict__ w = a.w_down + (int64_t) (o0 + ob) * d + lane;
+        for (int u = 0; u < PER; ++u)
+            if (!GUARD || tid + 256 * u < n4) *(v4f_t *) (xs_t + 4 * (tid + 256 * u)) = x[u];
+        const float st_l = st;
+        lds_sync();
+        if (t0 + (int) gridDim.y * RD_T < a.T) load_x(t0 + gridDim.y * RD_T);
 #pragma unroll
-            for (int j = 0; j < NI; ++j) wv[ob][j] = !GUARD || lane + 64 * j < d ? w[64 * j] : 0.0f;
-            b[ob] = a.b_down[o0 + ob];
-        }
-        // the state terms of the group's (token, output) pairs, lane tt * OB + ob, read back by readlane
-        float st_l = 0.0f;
-        if (eda && lane < RD_T * OB) {
-            const int o = o0 + lane % OB;
-            st_l = a.state_in[(int64_t) (t0 + min(lane / OB, nt - 1)) * a.rd + o] * a.eda[o];
-        }
-#pragma unroll 2
-        for (int tt = 0; tt < RD_T; ++tt) {
-            const int t = t0 + min(tt, nt - 1);
-            const float * xr = xs_t + (tt * 64 + lane) * S;
-            float acc[OB];
+        for (int h = 0; h < NH; ++h) {
+            if (NH > 1) load_w(h);
+#pragma unroll 1
+            for (int tt = 0; tt < nt; ++tt) {
+                const float * xr = xs_t + tt * d + 4 * p;
+                v4f_t c = (v4f_t) {0.0f, 0.0f, 0.0f, 0.0f};
+                if (h) c = part[256 * tt];
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ob] = 0.0f;
-#pragma unroll
-            for (int j4 = 0; j4 < NI / 4; ++j4) {
-                const float4 xv = *(const float4 *) (xr + 4 * j4);
-                const float xx[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj) {
-                    const int j = 4 * j4 + jj;
-                    if (!GUARD || lane + 64 * j < d) {
-#pragma unroll
-                        for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_fmaf(wv[ob][j], xx[jj], acc[ob]);
+                for (int j = 0; j < JH; ++j) {
+                    const int i = 64 * (h * JH + j);
+                    if (!GUARD || i + 4 * p < d) {
+                        const v4f_t xv = *(const v4f_t *) (xr + i);
+                        c.x = __builtin_fmaf(wv[j].x, xv.x, c.x);
+                        c.y = __builtin_fmaf(wv[j].y, xv.y, c.y);
+                        c.z = __builtin_fmaf(wv[j].z, xv.z, c.z);
+                        c.w = __builtin_fmaf(wv[j].w, xv.w, c.w);
                     }
                 }
-            }
+                if constexpr (!GUARD && JH > 8) {
+                    // eight reads ahead of the chains (left alone, each read is waited for by itself)
+                    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);        // LDS reads
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) {
-                const float st = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, st_l), tt * OB + ob));
-                float v = wave_tree_f(acc[ob]) + b[ob];
-                if (eda) v = v + st;
-                if (lane == 0 && tt < nt) a.rh[(int64_t) t * a.rd + o0 + ob] = v;
+                    for (int j = 8; j < JH; ++j) {
+                        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);      // VALU
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x2, 32, 0);
+                }
+                if (h + 1 < NH) { part[256 * tt] = c; continue; }
+                // wave_tree_f's additions: chain i + chain i + 32, + 16, + 8, + 4 (lanes p + 8 .. p + 1), + 2, + 1
+                float t4[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float v = t4[k];
+                    v = v + dpp_f<DPP_ROW_SHL + 8>(v);
+                    v = v + dpp_f<DPP_ROW_SHL + 4>(v);
+                    v = v + dpp_f<DPP_ROW_SHL + 2>(v);
+                    t4[k] = v + dpp_f<DPP_ROW_SHL + 1>(v);
+                }
+                float v = ((t4[0] + t4[2]) + (t4[1] + t4[3])) + b;
+                if (eda) v = v + __shfl(st_l, (lane & 48) + tt, 64);
+                if (p == 0) a.rh[(int64_t) (t0 + tt) * a.rd + o] = v;
             }
         }
+        lds_sync();                                                  // every wave has read the tile
     }
 }
 
