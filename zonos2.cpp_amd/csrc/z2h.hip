@@ -35,7 +35,9 @@ extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, false, true>(
 extern template __global__ void k_gemv_split<WF_Q8_0, true, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT, false, true>(GemvArgs);
 extern template __global__ void k_gemv_split<WF_Q8_0, false, MT_G, true, true>(GemvArgs);
-// the Q8_0 and Q6_K GEMMs, instantiated in z2h_wide.hip
+// the quantized GEMMs, instantiated in z2h_wide.hip
+extern template __global__ void k_gemm_q4k<true>(GemmArgs);
+extern template __global__ void k_gemm_q4k<false>(GemmArgs);
 extern template __global__ void k_gemm_q80<true, 1>(GemmArgs);
 extern template __global__ void k_gemm_q80<true, 2>(GemmArgs);
 extern template __global__ void k_gemm_q80<false, 1>(GemmArgs);
@@ -627,14 +629,16 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 //                top-4 of 32: Q6_K gate/up 38 us against 52, down 22 against 32; 48 rows, 6 routes: level
 //                before the sort launch is counted).
 constexpr int GEMM_MIN_ROWS = 65;
+// (k_gemm_q4k's activation offsets are 32-bit)
+bool gemm_q4k_ok(const DevMat & m, int64_t items) { return items * m.nsb * 256 < (int64_t) 1 << 32; }
 bool use_gemm(const z2h_ctx * ctx, const DevMat & m, int n_tok) {
     if (!m.m16) return m.type == Z2H_F16;
-    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, n_tok);
     return n_tok > 2 && 2ll * ((m.tiles + 3) / 4) * ((n_tok + 15) / 16) > ctx->n_cu;
 }
 bool use_gemm_experts(const DevMat & m, int n_tok, int k, int E) {
     if (!m.m16) return m.type == Z2H_F16;
-    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS;
+    if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, (int64_t) n_tok * k);
     return n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
 }
 // gate and up fused with SwiGLU in one GEMM launch: same type, layout and shape
@@ -661,9 +665,9 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
     a.r_off = g.r_off; a.r_perm = g.r_perm; a.act = g.act;
     a.out = g.out[0]; a.out_ld = g.out_ld; a.epi = g.epi; a.cap = g.cap; a.route_w = g.route_w;
     if (m0.type == Z2H_Q4_K) {
-        const dim3 grid(dual ? (m0.tiles + 3) / 4 : (m0.tiles + 7) / 8, gemm_slots(a.grouped, a.n_tok, a.k, a.E, GM_T));
-        if (dual) KL(k_gemm_q4k<true>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
-        else KL(k_gemm_q4k<false>, grid, dim3(256), gemm_q4k_lds(), ctx->stream, a);
+        const dim3 grid(dual ? (m0.tiles + 3) / 4 : (m0.tiles + 7) / 8, gemm_slots(a.grouped, a.n_tok, a.k, a.E, Q4_T));
+        if (dual) KL(k_gemm_q4k<true>, grid, dim3(256), gemm_q4k_lds, ctx->stream, a);
+        else KL(k_gemm_q4k<false>, grid, dim3(256), gemm_q4k_lds, ctx->stream, a);
     } else if (m0.m16) {
         // the tallest token tile that is half full on average and leaves at least two blocks per compute
         // unit (grouped launches fill about routes / GT + E / 2 tile slots): 333 rows of Q8_0 W_o 11.0 us

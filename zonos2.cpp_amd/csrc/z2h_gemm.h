@@ -1,19 +1,19 @@
 // z2h_gemm.h — MFMA GEMMs for the passes with many rows per weight tile: prefill chunks and mixed
 // prefill + decode passes (mul_mat / mul_mat_id over a whole batch, src/zonos2-graph.cpp:107-111,
-// 175, 179-185, 222-231). A block owns a tile of output rows x GM_T token (or route) rows and reads
-// each weight byte of its rows once for all GM_T rows; the activations of the tile are staged in LDS
+// 175, 179-185, 222-231). A block owns a tile of output rows x GT token (or route) rows and reads
+// each weight byte of its rows once for all GT rows; the activations of the tile are staged in LDS
 // one 256-column superblock at a time (double-buffered, the next superblock's loads in flight during
 // the current one's products). Grouped launches (experts) take their tiles from the route grouping
 // (k_route_sort's offsets and permutation): tile slots are numbered expert by expert, ceil(routes /
-// GM_T) per expert, and blocks whose slot is past the last tile exit.
+// GT) per expert, and blocks whose slot is past the last tile exit.
 //
-//   k_gemm_q4k   Q4_K weights (m16 layout) x Q8_K activations on int8 MFMA (v_mfma_i32_16x16x64_i8).
+//   k_gemm_q4k   Q4_K weights (m16 layout) x Q8_K activations on int8 MFMA (v_mfma_i32_32x32x32_i8).
 //                A Q4_K sub-block's 6-bit scale sc is split as 8 * (sc >> 3) + (sc & 7); the weights'
 //                4-bit values times each part stay below 106, so two int8 products over the whole
 //                superblock give sum_j sc_j * dot_j = 8 * hi + lo exactly, with no per-sub-block
-//                scaling of MFMA results. The min term sum_j m_j * bsum_j (bsum = the activation's
-//                sum over sub-block j) is one f16 MFMA on exact operands (bsum split as 64 * hi + lo),
-//                exact in fp32. Per superblock: acc = fma(dx, fma(d, isum, -dmin * msum), acc), the
+//                scaling of MFMA results. The min term sum_g m_g * bsum_g (bsum = the activation's
+//                sums of 16, g's min that of its sub-block) is one f16 MFMA on exact operands, exact
+//                in fp32. Per superblock: acc = fma(dx, fma(d, isum, -dmin * msum), acc), the
 //                fold of the Q4_K GEMVs, so a row's result is the same bits at any batch width.
 //   k_gemm_f16   F16 weights (t64 layout) x f16 activations on v_mfma_f32_16x16x32_f16, fp32
 //                accumulation; the weight fragments stream straight from HBM into a register ring of
@@ -23,10 +23,6 @@
 
 namespace z2d {
 
-constexpr int GM_T = 64;                 // token (route) rows per block tile
-constexpr int GM_QP = 256 + 8;           // LDS pitch of a row's int8 superblock (bytes): 66 dwords, so the
-                                         // 8-byte A reads of 16 rows fall in distinct banks
-constexpr int GM_SP = 10;                // LDS pitch (dwords) of a row's 8 sub-block sum pairs (same reason)
 constexpr int GM_HP = 256 + 8;           // LDS pitch of a row's f16 superblock (halves)
 
 typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
@@ -82,7 +78,8 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs & a, int slot, int & e,
     return false;
 }
 
-// Tile rows -> activation rows (s_row, the last valid row repeated past nt) and output row indices.
+// Tile rows -> activation rows (s_row, the last valid row repeated past nt), output row indices (s_out) and,
+// behind those, the rows' route weights (EPI_ROUTE_W): 3 GT words of LDS.
 template <int GT>
 __device__ __forceinline__ void gemm_rows(const GemmArgs & a, int e, int c0, int nt, int * s_row, int * s_out) {
     const int tid = threadIdx.x;
@@ -91,12 +88,14 @@ __device__ __forceinline__ void gemm_rows(const GemmArgs & a, int e, int c0, int
         const int it = a.grouped ? a.r_perm[a.r_off[e] + c0 + t] : c0 + t;
         s_out[tid] = it;
         s_row[tid] = a.grouped && !a.act_by_route ? it / a.k : it;
+        ((float *) s_out)[GT + tid] = a.epi == EPI_ROUTE_W ? a.route_w[it] : 0.0f;
     }
 }
 
-__device__ __forceinline__ float gemm_epi(const GemmArgs & a, float y, int it) {
+// rw: the row's route weight
+__device__ __forceinline__ float gemm_epi(const GemmArgs & a, float y, float rw) {
     if (a.epi == EPI_SOFTCAP) return z_softcap(y, a.cap);
-    if (a.epi == EPI_ROUTE_W) return y * a.route_w[it];
+    if (a.epi == EPI_ROUTE_W) return y * rw;
     return y;
 }
 
@@ -105,68 +104,95 @@ __device__ __forceinline__ float gemm_epi(const GemmArgs & a, float y, int it) {
 template <bool DUAL, int NG, int TS>
 __device__ __forceinline__ void gemm_store(const GemmArgs & a, const float (&acc)[NG][TS][4], const int (&grp)[NG], int lane,
                                            int nt, const int * s_out) {
+    constexpr int GT = 16 * TS;
 #pragma unroll
-    for (int ts = 0; ts < TS; ++ts)
+    for (int ts = 0; ts < TS; ++ts) {
+        const int t0 = ts * 16 + 4 * (lane >> 4);
+        const v4i_t oi = *(const v4i_t *) (s_out + t0);
+        const v4f_t rw = *(const v4f_t *) ((const float *) s_out + GT + t0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int t = ts * 16 + 4 * (lane >> 4) + i;
-            if (t >= nt) continue;
-            const int it = s_out[t];
-            float * o = a.out + (int64_t) it * a.out_ld;
+            if (t0 + i >= nt) continue;
+            float * o = a.out + (int64_t) oi[i] * a.out_ld;
 #pragma unroll
             for (int x = 0; x < (DUAL ? 1 : NG); ++x) {
                 const int row = grp[x] * 16 + (lane & 15);
                 if (grp[x] >= a.tiles || row >= a.rows) continue;
                 if constexpr (DUAL) o[row] = acc[1][ts][i] * z_silu(acc[0][ts][i]);
-                else o[row] = gemm_epi(a, acc[x][ts][i], it);
+                else o[row] = gemm_epi(a, acc[x][ts][i], rw[i]);
             }
         }
+    }
 }
 
 // ------------------------------------------------------------------ Q4_K x Q8_K
-// One superblock of GM_T activation rows in registers (GM_T / 16 x 16 B of values, GM_T / 32 sub-block
-// sum pairs and the block scale per thread), then in LDS: values [GM_T][GM_QP], sums as f16 pairs
-// (hi, lo) with sum = 64 * hi + lo [GM_T][GM_SP], scales [GM_T].
-struct GmQ8K { u32x4 v[GM_T / 16]; uint32_t s[GM_T / 32]; float dx; };
+// A block owns 128 weight rows (DUAL: 64 of gate and the same 64 of up), 32 per wave, x GT = 32 TS
+// token rows. The wave's 32 rows are one B operand of v_mfma_i32_32x32x32_i8: lane l has row l % 32
+// (16-row group (l / 16) & 1; DUAL: gate, up) and columns 32 j + 16 h .. + 15 of sub-block j, h = l / 32.
+//
+// Bounded by issue, not by memory (L2 hits at 80%, HBM idle): the vector unit (the weights' unpacking, 22
+// instructions per sub-block, and the fp32 fold, 5 per output) and the matrix unit are busy 60% and 34%
+// of the time. So the unpacking of sub-block j + 1 sits between the products of sub-block j (the group
+// barriers), 32 x 32 products take half the LDS reads and min-term products of 16 x 16 ones, the min term
+// takes the sums of 16 as they are, the staging has no address arithmetic, and a SwiGLU is formed once per output
+// by splitting the tokens over the gate and up lanes. A tile of up to 32 rows takes one product per sub-block.
+// Measured: 2088 rows, top-4 of 32, 2048 x 1536: gate/up 201 -> 167 us, down 129 -> 96; QKV 58 -> 48, W_o 46 ->
+// 38; 1024 rows 115 -> 95, 71 -> 54, 32 -> 27, 23 -> 19. Tiles of 96 and 128 rows (2 waves per SIMD still; 128
+// spills) 179 and 250 us for gate/up, of 32 rows only 178 (three waves per SIMD, twice the L2 reads).
+constexpr int Q4_SP = 12;                // LDS pitch (dwords) of a row's 16 f16 sums: 16 rows' 16-byte reads
+                                         // fall in distinct banks
+typedef int v16i_t __attribute__((ext_vector_type(16)));
+typedef float v16f_t __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ void gm_load_q8k(GmQ8K & st, const ActBuf & act, int K, int sb, const int * s_row) {
-    const int tid = threadIdx.x;
+constexpr int Q4_T = 64;                 // token (route) rows per block tile: one or two products of 32
+// One superblock of 32 S activation rows: values [32 S][256 B], a row's 16-byte chunk c at slot c ^ (row % 16)
+// (16 rows' reads of one chunk fall in distinct banks), the 16 sums of 16 as f16 (|sum| <= 2032, exact)
+// [32 S][Q4_SP], the scales [32 S].
+constexpr int q4_buf(int S) { return 32 * S * (256 + 4 * Q4_SP + 4); }
+constexpr size_t gemm_q4k_lds = 2 * q4_buf(2) + 3 * Q4_T * 4;
+
+// A thread's share of a superblock: 16-byte items of values, pairs of sums, one scale, at 32-bit byte
+// offsets (the host keeps rows x K below 2^32) from the superblock's uniform base: no address arithmetic.
+template <int S>
+struct Q4Stage {
+    uint32_t ov[2 * S], os[S], od;
+    u32x4 v[2 * S];
+    uint32_t s[S];
+    float dx;
+};
+template <int S>
+__device__ __forceinline__ void q4_rows(Q4Stage<S> & st, int K, const int * s_row) {
+    const uint32_t tid = threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < GM_T / 16; ++j) {
-        const int i = tid + 256 * j, r = i >> 4, c = i & 15;
-        st.v[j] = *(const u32x4 *) (act.q + (int64_t) s_row[r] * K + sb * 256 + c * 16);
-    }
+    for (int j = 0; j < 2 * S; ++j) st.ov[j] = (uint32_t) s_row[16 * j + (tid >> 4)] * (uint32_t) K + (tid & 15) * 16;
 #pragma unroll
-    for (int j = 0; j < GM_T / 32; ++j) {
-        const int i = tid + 256 * j, r = i >> 3, jj = i & 7;
-        st.s[j] = *(const uint32_t *) (act.bs + (int64_t) s_row[r] * (K / 16) + sb * 16 + 2 * jj);
-    }
-    st.dx = act.d256[(int64_t) s_row[tid & (GM_T - 1)] * (K / 256) + sb];
+    for (int j = 0; j < S; ++j) st.os[j] = (uint32_t) s_row[32 * j + (tid >> 3)] * (uint32_t) (K / 8) + (tid & 7) * 4;
+    st.od = (uint32_t) s_row[tid & (32 * S - 1)] * (uint32_t) (K / 64);
 }
-
-__device__ __forceinline__ void gm_store_q8k(const GmQ8K & st, int8_t * sq, uint32_t * ss, float * sdx) {
-    const int tid = threadIdx.x;
+template <int S>
+__device__ __forceinline__ void q4_load(Q4Stage<S> & st, const ActBuf & act, int sb) {
+    const uint8_t * q = (const uint8_t *) act.q + (size_t) sb * 256, * bs = (const uint8_t *) act.bs + (size_t) sb * 32,
+                  * d = (const uint8_t *) act.d256 + (size_t) sb * 4;
 #pragma unroll
-    for (int j = 0; j < GM_T / 16; ++j) {
-        const int i = tid + 256 * j, r = i >> 4, c = i & 15;
-        uint2 * dst = (uint2 *) (sq + r * GM_QP + c * 16);            // 8-byte aligned rows
-        dst[0] = make_uint2(st.v[j].x, st.v[j].y);
-        dst[1] = make_uint2(st.v[j].z, st.v[j].w);
-    }
+    for (int j = 0; j < 2 * S; ++j) st.v[j] = *(const u32x4 *) (q + st.ov[j]);
 #pragma unroll
-    for (int j = 0; j < GM_T / 32; ++j) {
-        const int i = tid + 256 * j;
-        const int s = (int) (int16_t) (st.s[j] & 0xffffu) + (int) (int16_t) (st.s[j] >> 16);   // |s| <= 32 * 128
-        const _Float16 hi = (_Float16) (s >> 6), lo = (_Float16) (s & 63);
-        ss[(i >> 3) * GM_SP + (i & 7)] = (uint32_t) __builtin_bit_cast(uint16_t, hi) | ((uint32_t) __builtin_bit_cast(uint16_t, lo) << 16);
-    }
-    if (tid < GM_T) sdx[tid] = st.dx;
+    for (int j = 0; j < S; ++j) st.s[j] = *(const uint32_t *) (bs + st.os[j]);
+    st.dx = *(const float *) (d + st.od);
 }
-
-// The B operands of one m16 unit (16 rows x 256 columns) for the lane's row and k-slice: for each
-// pair of sub-blocks (2s, 2s+1) the 16 weight values times the high and the low part of their
-// sub-block scales, the f16 operand of the min term, and the row's d / dmin.
-struct GmQ4Unit { v4i_t bh[4], bl[4]; v4h_t bm; float d, dmin; };
+template <int S>
+__device__ __forceinline__ void q4_store(const Q4Stage<S> & st, char * buf) {
+    const int tid = threadIdx.x, c = (tid & 15) ^ (tid >> 4);         // (row % 16 = tid / 16)
+    uint32_t * ss = (uint32_t *) (buf + 32 * S * 256);
+    float * sdx = (float *) (ss + 32 * S * Q4_SP);
+#pragma unroll
+    for (int j = 0; j < 2 * S; ++j) *(u32x4 *) (buf + (16 * j + (tid >> 4)) * 256 + c * 16) = st.v[j];
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+        const _Float16 lo = (_Float16) (int16_t) (st.s[j] & 0xffffu), hi = (_Float16) (int16_t) (st.s[j] >> 16);
+        ss[(32 * j + (tid >> 3)) * Q4_SP + (tid & 7)] = (uint32_t) __builtin_bit_cast(uint16_t, lo) | ((uint32_t) __builtin_bit_cast(uint16_t, hi) << 16);
+    }
+    sdx[tid & (32 * S - 1)] = st.dx;                                   // (several threads store the same value)
+}
 
 __device__ __forceinline__ uint32_t gm_mul_bytes(uint32_t x, uint32_t s) {
     // four byte lanes (each <= 15) times s <= 7: two 16-bit products per half, no carry across bytes
@@ -174,131 +200,149 @@ __device__ __forceinline__ uint32_t gm_mul_bytes(uint32_t x, uint32_t s) {
     return __builtin_bit_cast(uint32_t, r);
 }
 
-__device__ __forceinline__ void gm_prep_q4k(const uint4 & q0, const uint4 & q1, const uint4 & hd, int lane, GmQ4Unit & u) {
-    const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-    // 6-bit scales / mins of sub-blocks 0-3 and 4-7 (GGUF K-quant packing)
-    const uint32_t sc03 = hd.y & 0x3f3f3f3fu;
-    const uint32_t sc47 = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
-    const uint32_t mn03 = hd.z & 0x3f3f3f3fu;
-    const uint32_t mn47 = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
+// The B operands of sub-block j for the lane's row and column half: its 16 weight values times the high and
+// the low part of the sub-block's scale (sc03, sc47: the row's 8 scales). raw[2 c + e]: chunk c of the m16
+// unit's k-slice 2 h + e.
+struct Q4B { v4i_t hi, lo; };
+__device__ __forceinline__ Q4B q4_prep(const u32x4 (&raw)[4], uint32_t sc03, uint32_t sc47, int j) {
+    const int p = j >> 1;                                            // sub-blocks 2p (low nibbles) and 2p + 1
+    const u32x4 & r0 = raw[2 * (p >> 1)], & r1 = raw[2 * (p >> 1) + 1];
+    const uint32_t w[4] = {(p & 1) ? r0.z : r0.x, (p & 1) ? r0.w : r0.y, (p & 1) ? r1.z : r1.x, (p & 1) ? r1.w : r1.y};
+    const uint32_t sc = (j < 4 ? sc03 : sc47) >> (8 * (j & 3)), sh = (sc >> 3) & 7u, sl = sc & 7u;
+    Q4B b;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const uint32_t sc = s < 2 ? sc03 : sc47;
-        const int j0 = 2 * (s & 1);                                  // byte of sub-block 2s in sc
-        const uint32_t h0 = (sc >> (8 * j0 + 3)) & 7u, l0 = (sc >> (8 * j0)) & 7u;
-        const uint32_t h1 = (sc >> (8 * j0 + 11)) & 7u, l1 = (sc >> (8 * j0 + 8)) & 7u;
-        const uint32_t a0 = w[2 * s] & 0x0f0f0f0fu, a1 = w[2 * s + 1] & 0x0f0f0f0fu;              // sub-block 2s
-        const uint32_t b0 = (w[2 * s] >> 4) & 0x0f0f0f0fu, b1 = (w[2 * s + 1] >> 4) & 0x0f0f0f0fu;  // sub-block 2s+1
-        u.bh[s] = (v4i_t) {(int) gm_mul_bytes(a0, h0), (int) gm_mul_bytes(a1, h0), (int) gm_mul_bytes(b0, h1), (int) gm_mul_bytes(b1, h1)};
-        u.bl[s] = (v4i_t) {(int) gm_mul_bytes(a0, l0), (int) gm_mul_bytes(a1, l0), (int) gm_mul_bytes(b0, l1), (int) gm_mul_bytes(b1, l1)};
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t v = ((j & 1) ? w[i] >> 4 : w[i]) & 0x0f0f0f0fu;
+        b.hi[i] = (int) gm_mul_bytes(v, sh);
+        b.lo[i] = (int) gm_mul_bytes(v, sl);
     }
-    const int q = lane >> 4;
-    const uint32_t mm = (q < 2 ? mn03 : mn47) >> (16 * (q & 1));
-    const float ma = (float) (mm & 0xffu), mb = (float) ((mm >> 8) & 0xffu);
-    u.bm = (v4h_t) {(_Float16) (64.0f * ma), (_Float16) ma, (_Float16) (64.0f * mb), (_Float16) mb};
-    u.d = h2f(hd.x & 0xffffu);
-    u.dmin = h2f(hd.x >> 16);
+    return b;
 }
 
-// grid: x = row blocks (DUAL: 4 16-row groups of gate and up, each wave one group of both; else 8
-// groups, two per wave), y = tile slots. 256 threads; dynamic LDS gemm_q4k_lds().
-__host__ __device__ inline size_t gemm_q4k_lds() { return 2 * (size_t) (GM_T * GM_QP + GM_T * GM_SP * 4 + GM_T * 4) + 2 * GM_T * 4; }
+// One block tile of up to 32 S rows.
+template <bool DUAL, int S>
+__device__ __forceinline__ void q4_block(const GemmArgs & a, char * smem, const int * s_row, const int * s_out, int nt,
+                                         int grp, const u32x4 * wl, const u32x4 * wh, u32x4 (&raw)[4], u32x4 & hd) {
+    constexpr int BUF = q4_buf(S);
+    const int tid = threadIdx.x, lane = tid & 63, K = a.nsb * 256, h = lane >> 5, x = (lane >> 4) & 1;
+    Q4Stage<S> st;
+    q4_rows(st, K, s_row);
+    q4_load(st, a.act, 0);
+    q4_store(st, smem);
+    lds_sync();
+    float acc[S][16] = {};
+    for (int sb = 0; sb < a.nsb; ++sb) {
+        const char * buf = smem + (sb & 1) * BUF;
+        char * nb = smem + ((sb + 1) & 1) * BUF;
+        const int nx = min(sb + 1, a.nsb - 1);                       // (the last superblock re-reads itself)
+        q4_load(st, a.act, nx);
+        // the row's 6-bit scales / mins of sub-blocks 0-3 and 4-7 (GGUF K-quant packing), d, dmin; the lane's
+        // 8 sums of the min term belong to sub-blocks 4h .. 4h + 3
+        const uint32_t sc03 = hd.y & 0x3f3f3f3fu, sc47 = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
+        const uint32_t mm = h ? ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3f3f3f3fu;
+        const float d = h2f(hd.x & 0xffffu), dmin = h2f(hd.x >> 16);
+        v16i_t ch[S], cl[S];
+#pragma unroll
+        for (int ts = 0; ts < S; ++ts) ch[ts] = cl[ts] = (v16i_t) {};
+        // sub-block j + 1's operands are read and unpacked between sub-block j's products
+        auto load_a = [&](int j, v4i_t (&A)[S]) {
+#pragma unroll
+            for (int ts = 0; ts < S; ++ts)
+                A[ts] = *(const v4i_t *) (buf + (ts * 32 + (lane & 31)) * 256 + (((2 * j + h) ^ (lane & 15)) << 4));
+        };
+        v4i_t A[2][S];
+        Q4B B[2];
+        load_a(0, A[0]);
+        B[0] = q4_prep(raw, sc03, sc47, 0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j < 7) {
+                load_a(j + 1, A[(j + 1) & 1]);
+                B[(j + 1) & 1] = q4_prep(raw, sc03, sc47, j + 1);
+            }
+            if (j == 3) { raw[0] = wl[(size_t) nx * 144]; raw[1] = wl[(size_t) nx * 144 + 16]; hd = wh[(size_t) nx * 144]; }
+            if (j == 7) { raw[2] = wl[(size_t) nx * 144 + 64]; raw[3] = wl[(size_t) nx * 144 + 80]; }
+#pragma unroll
+            for (int ts = 0; ts < S; ++ts) {
+                ch[ts] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j & 1][ts], B[j & 1].hi, ch[ts], 0, 0, 0);
+                cl[ts] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j & 1][ts], B[j & 1].lo, cl[ts], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, S, 0);    // LDS reads
+#pragma unroll
+            for (int i = 0; i < 2 * S; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x2, 10 / S, 0);   // VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        v8h_t bm;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bm[2 * i] = bm[2 * i + 1] = (_Float16) (float) ((mm >> (8 * i)) & 0xffu);
+#pragma unroll
+        for (int ts = 0; ts < S; ++ts) {
+            const uint32_t * sp = (const uint32_t *) (buf + 32 * S * 256) + (ts * 32 + (lane & 31)) * Q4_SP + 4 * h;
+            const float * dxp = (const float *) (buf + 32 * S * (256 + 4 * Q4_SP)) + ts * 32 + 4 * h;
+            const v16f_t M = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const v8h_t *) sp, bm, (v16f_t) {}, 0, 0, 0);
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                const v4f_t dx = *(const v4f_t *) (dxp + 8 * i4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    // the Q4_K unit value and fold of m16_unit / m16_fold (same operations)
+                    const int c = 4 * i4 + i;
+                    const float f = (float) ((ch[ts][c] << 3) + cl[ts][c]);
+                    acc[ts][c] = __builtin_fmaf(dx[i], __builtin_fmaf(d, f, -(dmin * M[c])), acc[ts][c]);
+                }
+            }
+        }
+        q4_store(st, nb);
+        lds_sync();
+    }
+    const int row = grp * 16 + (lane & 15);
+    const bool st_ok = grp < a.tiles && row < a.rows;
+#pragma unroll
+    for (int i8 = 0; i8 < 4 * S; ++i8) {
+        const int ts = i8 >> 2, i4 = i8 & 3, t0 = ts * 32 + 8 * i4 + 4 * h;
+        if (32 * ts >= nt) break;                                    // (uniform)
+        if constexpr (DUAL) {
+            // lanes x = 0 hold gate, the lanes 16 above the same rows of up: one swap leaves the gates of
+            // tokens i (x = 0) and i + 1 (x = 1) in one register and their ups in the other
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, acc[ts][4 * i4 + i]),
+                                                                 __builtin_bit_cast(unsigned, acc[ts][4 * i4 + i + 1]), false, false);
+                const unsigned gb = sw[0], ub = sw[1];
+                const float y = __builtin_bit_cast(float, ub) * z_silu(__builtin_bit_cast(float, gb));
+                if (st_ok && t0 + i + x < nt) a.out[(int64_t) s_out[t0 + i + x] * a.out_ld + row] = y;
+            }
+        } else {
+            const v4i_t oi = *(const v4i_t *) (s_out + t0);
+            const v4f_t rw = *(const v4f_t *) ((const float *) s_out + Q4_T + t0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (st_ok && t0 + i < nt) a.out[(int64_t) oi[i] * a.out_ld + row] = gemm_epi(a, acc[ts][4 * i4 + i], rw[i]);
+        }
+    }
+}
 
+// grid: x = blocks of eight 16-row groups (DUAL: four of gate and of up), y = tile slots. 256 threads;
+// dynamic LDS gemm_q4k_lds.
 template <bool DUAL>
 __global__ void __launch_bounds__(256, 2) k_gemm_q4k(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int BUF = GM_T * GM_QP + GM_T * GM_SP * 4 + GM_T * 4;
-    int * s_row = (int *) (smem + 2 * BUF), * s_out = s_row + GM_T;
+    int * s_row = (int *) (smem + 2 * q4_buf(2)), * s_out = s_row + Q4_T;
     int e, c0, nt;
-    if (!gemm_tile<GM_T>(a, blockIdx.y, e, c0, nt)) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, K = a.nsb * 256;
-    gemm_rows<GM_T>(a, e, c0, nt, s_row, s_out);
-    // the wave's two 16-row units
-    const int gA = DUAL ? blockIdx.x * 4 + wave : (blockIdx.x * 4 + wave) * 2, gB = DUAL ? gA : gA + 1;
-    const bool has = gA < a.tiles;
-    const uint8_t * wA = a.w[0] + (int64_t) e * a.mat_bytes + (size_t) (has ? gA : 0) * a.nsb * 2304;
-    const uint8_t * wB = (DUAL ? a.w[1] : a.w[0]) + (int64_t) e * a.mat_bytes + (size_t) (gB < a.tiles ? gB : 0) * a.nsb * 2304;
-    uint4 raw[2][3];
-    auto load_w = [&](int sb) {
-        const uint4 * pa = (const uint4 *) (wA + (size_t) sb * 2304), * pb = (const uint4 *) (wB + (size_t) sb * 2304);
-        raw[0][0] = pa[lane]; raw[0][1] = pa[64 + lane]; raw[0][2] = pa[128 + (lane & 15)];
-        raw[1][0] = pb[lane]; raw[1][1] = pb[64 + lane]; raw[1][2] = pb[128 + (lane & 15)];
-    };
-    if (has) load_w(0);
-    lds_sync();                                                      // s_row
-    GmQ8K st;
-    gm_load_q8k(st, a.act, K, 0, s_row);
-    gm_store_q8k(st, (int8_t *) smem, (uint32_t *) (smem + GM_T * GM_QP), (float *) (smem + GM_T * GM_QP + GM_T * GM_SP * 4));
+    if (!gemm_tile<Q4_T>(a, blockIdx.y, e, c0, nt)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), x = (lane >> 4) & 1;
+    // the lane's 16-row group (lanes past the last group read group 0 and store nothing) and its first unit
+    const int grp = DUAL ? blockIdx.x * 4 + wave : (blockIdx.x * 4 + wave) * 2 + x;
+    const u32x4 * w = (const u32x4 *) ((DUAL && x ? a.w[1] : a.w[0]) + (int64_t) e * a.mat_bytes + (size_t) (grp < a.tiles ? grp : 0) * a.nsb * 2304);
+    const u32x4 * wl = w + 32 * (lane >> 5) + (lane & 15), * wh = w + 128 + (lane & 15);
+    u32x4 raw[4] = {wl[0], wl[16], wl[64], wl[80]}, hd = wh[0];
+    gemm_rows<Q4_T>(a, e, c0, nt, s_row, s_out);
     lds_sync();
-    float acc[2][GM_T / 16][4] = {};
-    const v4i_t zi = {0, 0, 0, 0};
-    const v4f_t zf = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int q = lane >> 4;
-    for (int sb = 0; sb < a.nsb; ++sb) {
-        char * buf = smem + (sb & 1) * BUF;
-        const int8_t * sq = (const int8_t *) buf;
-        const uint32_t * ss = (const uint32_t *) (buf + GM_T * GM_QP);
-        const float * sdx = (const float *) (buf + GM_T * GM_QP + GM_T * GM_SP * 4);
-        const bool more = sb + 1 < a.nsb;
-        if (more) gm_load_q8k(st, a.act, K, sb + 1, s_row);
-        if (has) {
-            GmQ4Unit u[2];
-            gm_prep_q4k(raw[0][0], raw[0][1], raw[0][2], lane, u[0]);
-            gm_prep_q4k(raw[1][0], raw[1][1], raw[1][2], lane, u[1]);
-            if (more) load_w(sb + 1);
-#pragma unroll
-            for (int ts = 0; ts < GM_T / 16; ++ts) {
-                const int r = ts * 16 + (lane & 15);
-                const int8_t * ap = sq + r * GM_QP + 8 * q;
-                v4i_t A[4];
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const uint2 lo = *(const uint2 *) (ap + 64 * s), hi = *(const uint2 *) (ap + 64 * s + 32);
-                    A[s] = (v4i_t) {(int) lo.x, (int) lo.y, (int) hi.x, (int) hi.y};
-                }
-                const v4h_t As = *(const v4h_t *) (ss + r * GM_SP + 2 * q);
-                const v4f_t dx = *(const v4f_t *) (sdx + ts * 16 + 4 * q);
-#pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    v4i_t ch = zi, cl = zi;
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[s], u[x].bh[s], ch, 0, 0, 0);
-                        cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[s], u[x].bl[s], cl, 0, 0, 0);
-                    }
-                    const v4f_t S = __builtin_amdgcn_mfma_f32_16x16x16f16(As, u[x].bm, zf, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        // the Q4_K unit value and fold of m16_unit / m16_fold (same operations)
-                        const float f = (float) ((ch[i] << 3) + cl[i]);
-                        acc[x][ts][i] = __builtin_fmaf(dx[i], __builtin_fmaf(u[x].d, f, -(u[x].dmin * S[i])), acc[x][ts][i]);
-                    }
-                }
-            }
-        }
-        if (more) {
-            char * nb = smem + ((sb + 1) & 1) * BUF;
-            gm_store_q8k(st, (int8_t *) nb, (uint32_t *) (nb + GM_T * GM_QP), (float *) (nb + GM_T * GM_QP + GM_T * GM_SP * 4));
-        }
-        lds_sync();
-    }
-    if (!has) return;
-    const int row = gA * 16 + (lane & 15), rowB = gB * 16 + (lane & 15);
-#pragma unroll
-    for (int ts = 0; ts < GM_T / 16; ++ts)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int t = ts * 16 + 4 * q + i;
-            if (t >= nt) continue;
-            const int it = s_out[t];
-            float * o = a.out + (int64_t) it * a.out_ld;
-            if (DUAL) {
-                if (row < a.rows) o[row] = acc[1][ts][i] * z_silu(acc[0][ts][i]);
-            } else {
-                if (row < a.rows) o[row] = gemm_epi(a, acc[0][ts][i], it);
-                if (rowB < a.rows) o[rowB] = gemm_epi(a, acc[1][ts][i], it);
-            }
-        }
+    if (__builtin_amdgcn_readfirstlane(nt) > 32) q4_block<DUAL, 2>(a, smem, s_row, s_out, nt, grp, wl, wh, raw, hd);
+    else q4_block<DUAL, 1>(a, smem, s_row, s_out, nt, grp, wl, wh, raw, hd);
 }
 
 // ------------------------------------------------------------------ F16 x f16
@@ -333,7 +377,7 @@ __device__ __forceinline__ void gm_store_f16(const GmF16<TS> & st, int h, uint16
     }
 }
 
-__host__ __device__ inline size_t gemm_f16_lds(int ts) { return 2 * (size_t) (16 * ts) * GM_HP * 2 + 2 * (16 * ts) * 4; }
+__host__ __device__ inline size_t gemm_f16_lds(int ts) { return 2 * (size_t) (16 * ts) * GM_HP * 2 + 3 * (16 * ts) * 4; }
 
 template <bool DUAL, int NG, int TS>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16(GemmArgs a) {
@@ -427,7 +471,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f16(GemmArgs a) {
 #pragma unroll
                 for (int g = 0; g < NG; ++g) {
                     const int row = r0 + 16 * g + (lane & 15);
-                    if (row < a.rows) o[row] = gemm_epi(a, acc[g][ts][i], it);
+                    if (row < a.rows) o[row] = gemm_epi(a, acc[g][ts][i], ((const float *) s_out)[GT + t]);
                 }
             }
         }

@@ -78,7 +78,7 @@ __device__ __forceinline__ void gq_store_q80(const GqQ80<TS> & st, int8_t * sq, 
 }
 
 __host__ __device__ constexpr size_t gemm_q80_buf(int ts) { return (size_t) 16 * ts * (GQ_QP + 2 * GQ_DP); }
-__host__ __device__ inline size_t gemm_q80_lds(int ts) { return 2 * gemm_q80_buf(ts) + 2 * 16 * ts * 4; }
+__host__ __device__ inline size_t gemm_q80_lds(int ts) { return 2 * gemm_q80_buf(ts) + 3 * 16 * ts * 4; }
 
 // grid: x = blocks of four groups, y = tile slots; 256 threads
 template <bool DUAL, int TS>
@@ -240,7 +240,7 @@ __device__ __forceinline__ void gq_prep_q6k(uint32_t L, uint32_t hb, int sc, v4i
 }
 
 __host__ __device__ constexpr size_t gemm_q6k_buf(int ts) { return (size_t) 16 * ts * (GQ_QP + 4); }
-__host__ __device__ inline size_t gemm_q6k_lds(int ts) { return 2 * gemm_q6k_buf(ts) + 2 * 16 * ts * 4; }
+__host__ __device__ inline size_t gemm_q6k_lds(int ts) { return 2 * gemm_q6k_buf(ts) + 3 * 16 * ts * 4; }
 
 template <bool DUAL, int TS>
 __global__ void __launch_bounds__(256, 2) k_gemm_q6k(GemmArgs a) {
