@@ -20,7 +20,6 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <set>
 #include <memory>
 #include <string>
 #include <thread>
@@ -129,9 +128,10 @@ struct z2h_ctx {
     int Tstep = 0;                    // columns a step may list (n_slots); captures are sized for it
     int pch = 0;                      // prefill chunk rows (<= Tmax)
     int max_rows = 0;                 // requested row capacity (z2h_create_batch_rows)
-    int32_t * d_emb_map = nullptr;    // [Tmax] per-row embedding override
-    int32_t * d_head_rows = nullptr;  // [Tmax] rows of a mixed pass that get logits
-    int32_t * d_slot = nullptr, * d_npast = nullptr, * d_ids = nullptr; float * d_emb = nullptr;
+    // a pass's integer inputs, one block [(4 + W) Tmax] laid out like h_pin: slot | n_past | ids (W per row) |
+    // per-row embedding override | rows of a mixed pass that get logits
+    int32_t * d_slot = nullptr, * d_npast = nullptr, * d_ids = nullptr, * d_emb_map = nullptr, * d_head_rows = nullptr;
+    float * d_emb = nullptr;
     float * spk_io = nullptr;         // speaker projection: spk | lda out | proj out | delta
     float * res = nullptr, * res2 = nullptr, * cur = nullptr, * qkvg = nullptr, * wo_out = nullptr;
     float * part_o = nullptr, * part_ml = nullptr;
@@ -148,8 +148,8 @@ struct z2h_ctx {
     int * d_err = nullptr;
     int4 * d_tiles = nullptr;         // [items_max] attention tile entries of a kv_pre pass (k_attn_tile)
     int4 * h_tiles = nullptr;         // pinned staging for them
-    int32_t * h_pin = nullptr;        // pinned staging for step inputs
-    size_t h_pin_bytes = 0;
+    int32_t * h_pin = nullptr;        // pinned staging for step inputs (d_slot's block), then the error flag
+    std::vector<uint64_t> row_seen;   // z2h_step_mixed: one bit per cache row, all clear between calls
 
     // frame sampler: per-column settings, histories, draws and codes (device + pinned staging)
     SampleParams * d_sp = nullptr; int32_t * d_hist = nullptr, * d_hlen = nullptr, * d_codes = nullptr;
@@ -523,8 +523,7 @@ int alloc_scratch(z2h_ctx * ctx) {
     // act_y rows per token: the token's routes' FFN activations, or (the head's gathered rows) one
     // activation row of any matmul
     const size_t ypr = std::max((size_t) std::max(K, 1) * kpad(std::max(ff, 1)), (size_t) KM);
-    if ((rc = dalloc(ctx, &ctx->d_slot, T * 4, b)) || (rc = dalloc(ctx, &ctx->d_npast, T * 4, b)) ||
-        (rc = dalloc(ctx, &ctx->d_ids, (size_t) T * W * 4, b)) || (rc = dalloc(ctx, &ctx->d_emb, (size_t) T * d * 4, b)) ||
+    if ((rc = dalloc(ctx, &ctx->d_slot, (size_t) T * (4 + W) * 4, b)) || (rc = dalloc(ctx, &ctx->d_emb, (size_t) T * d * 4, b)) ||
         (rc = dalloc(ctx, &ctx->res, (size_t) T * d * 4, b)) || (rc = dalloc(ctx, &ctx->res2, (size_t) T * d * 4, b)) ||
         (rc = dalloc(ctx, &ctx->cur, (size_t) T * d * 4, b)) ||
         (rc = dalloc(ctx, &ctx->tmp_x, (size_t) T * d * 4, b)) ||
@@ -541,12 +540,10 @@ int alloc_scratch(z2h_ctx * ctx) {
         (rc = dalloc(ctx, &ctx->act_y.d256, (size_t) T * (ypr / 256) * 4, b)) ||
         (rc = dalloc(ctx, &ctx->act_y.bs, (size_t) T * (ypr / 16) * 2, b)) ||
         (rc = dalloc(ctx, &ctx->act_y.h, (size_t) T * ypr * 2, b)) ||
-        (rc = dalloc(ctx, &ctx->d_head_rows, (size_t) T * 4, b)) ||
         (rc = dalloc(ctx, &ctx->attn_o, (size_t) T * nh * hd * 4, b)) ||
         (rc = dalloc(ctx, &ctx->state, (size_t) hp.n_layer * T * rd * 4, b)) || (rc = dalloc(ctx, &ctx->state_ext, (size_t) T * rd * 4, b)) ||
         (rc = dalloc(ctx, &ctx->sel, (size_t) T * K * 4, b)) || (rc = dalloc(ctx, &ctx->wsel, (size_t) T * K * 4, b)) ||
         (rc = dalloc(ctx, &ctx->r_off, (size_t) (E + 1) * 4, b)) || (rc = dalloc(ctx, &ctx->r_perm, (size_t) T * K * 4, b)) ||
-        (rc = dalloc(ctx, &ctx->d_emb_map, (size_t) T * 4, b)) ||
         (rc = dalloc(ctx, &ctx->gu_g, (size_t) T * K * std::max(ff, 1) * 4, b)) || (rc = dalloc(ctx, &ctx->gu_u, (size_t) T * K * std::max(ff, 1) * 4, b)) ||
         (rc = dalloc(ctx, &ctx->eo, (size_t) T * K * d * 4, b)) ||
         (rc = dalloc(ctx, &ctx->logits, (size_t) T * hp.n_codebooks * hp.audio_vocab * 4, b)) ||
@@ -569,8 +566,8 @@ int alloc_scratch(z2h_ctx * ctx) {
     }
     if (hipHostMalloc((void **) &ctx->h_tiles, (size_t) 2 * ctx->items_max * sizeof(int4), hipHostMallocDefault) != hipSuccess)
         return seterr(ctx, Z2H_ENOMEM, "hipHostMalloc failed");
-    ctx->h_pin_bytes = (size_t) T * (4 + W) * 4;
-    if (hipHostMalloc((void **) &ctx->h_pin, ctx->h_pin_bytes, hipHostMallocDefault) != hipSuccess)
+    ctx->d_npast = ctx->d_slot + T; ctx->d_ids = ctx->d_npast + T; ctx->d_emb_map = ctx->d_ids + (size_t) T * W; ctx->d_head_rows = ctx->d_emb_map + T;
+    if (hipHostMalloc((void **) &ctx->h_pin, ((size_t) T * (4 + W) + 4) * 4, hipHostMallocDefault) != hipSuccess)
         return seterr(ctx, Z2H_ENOMEM, "hipHostMalloc failed");
     const int ncb = std::max(1, (int) hp.n_codebooks);
     if ((rc = dalloc(ctx, &ctx->d_sp, (size_t) T * sizeof(SampleParams), b)) ||
@@ -1468,10 +1465,21 @@ int launch_attn_fa(z2h_ctx * ctx, const AttnArgs & a, int grid) {
     return Z2H_OK;
 }
 
-int check_err_flag(z2h_ctx * ctx) {
-    int h = 0;
-    HIPX(hipMemcpy(&h, ctx->d_err, 4, hipMemcpyDeviceToHost));
-    if (h) {
+// One pinned upload of a pass's integer inputs, the first n ints of h_pin's block. Each copy costs about 8 us of
+// host time and queue time, so a pass makes one.
+int upload_inputs(z2h_ctx * ctx, size_t n) {
+    HIPX(hipMemcpyAsync(ctx->d_slot, ctx->h_pin, n * 4, hipMemcpyHostToDevice, ctx->stream));
+    return Z2H_OK;
+}
+
+// The end of a host call: n floats of logits to the host, the wait, and the error flag, copied ahead of the logits
+// so that it needs no wait of its own.
+int finish_pass(z2h_ctx * ctx, float * out, size_t n) {
+    int32_t * err = ctx->h_pin + (size_t) ctx->Tmax * (4 + ctx->W);
+    HIPX(hipMemcpyAsync(err, ctx->d_err, 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (out && n) HIPX(hipMemcpyAsync(out, ctx->logits, n * 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIPX(hipStreamSynchronize(ctx->stream));
+    if (*err) {
         HIPX(hipMemset(ctx->d_err, 0, 4));
         return seterr(ctx, Z2H_EINVAL, "token id out of range");
     }
@@ -1866,20 +1874,17 @@ int z2h_step(z2h_ctx * ctx, int T, const int32_t * slot_idx, const int32_t * n_p
     }
     HIPX(hipSetDevice(ctx->device));
     int32_t * hp_ = ctx->h_pin;
+    const size_t TM = ctx->Tmax;
     std::memcpy(hp_, slot_idx, (size_t) T * 4);
-    std::memcpy(hp_ + T, n_past, (size_t) T * 4);
-    if (ids) std::memcpy(hp_ + 2 * T, ids, (size_t) T * ctx->W * 4);
-    HIPX(hipMemcpyAsync(ctx->d_slot, hp_, (size_t) T * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPX(hipMemcpyAsync(ctx->d_npast, hp_ + T, (size_t) T * 4, hipMemcpyHostToDevice, ctx->stream));
-    if (ids) HIPX(hipMemcpyAsync(ctx->d_ids, hp_ + 2 * T, (size_t) T * ctx->W * 4, hipMemcpyHostToDevice, ctx->stream));
+    std::memcpy(hp_ + TM, n_past, (size_t) T * 4);
+    if (ids) std::memcpy(hp_ + 2 * TM, ids, (size_t) T * ctx->W * 4);
+    if (int rc = upload_inputs(ctx, ids ? 2 * TM + (size_t) T * ctx->W : TM + T)) return rc;
     if (emb) HIPX(hipMemcpyAsync(ctx->d_emb, emb, (size_t) T * ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
     ctx->resident_T = ctx->resident_last = 0;
     ctx->last_np.assign(n_past, n_past + T);
     if (int rc = step_internal(ctx, T, n_past, ids != nullptr)) return rc;
     const size_t nout = (size_t) T * ctx->hp.n_codebooks * ctx->hp.audio_vocab;
-    if (out_logits) HIPX(hipMemcpyAsync(out_logits, ctx->logits, nout * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    if (int rc = check_err_flag(ctx)) return rc;
+    if (int rc = finish_pass(ctx, out_logits, nout)) return rc;
     ctx->resident_last = T;
     return Z2H_OK;
 }
@@ -1975,27 +1980,24 @@ int z2h_prefill(z2h_ctx * ctx, int slot, const int32_t * ids, int n0, const floa
     for (int r0 = 0; r0 < n0; r0 += chunk) {
         const int T = std::min(chunk, n0 - r0);
         const bool last = r0 + T == n0;
-        int32_t * hp_ = ctx->h_pin;
-        for (int t = 0; t < T; ++t) { hp_[t] = slot; hp_[T + t] = r0 + t; }
-        std::memcpy(hp_ + 2 * T, ids + (size_t) r0 * W, (size_t) T * W * 4);
+        const size_t TM = ctx->Tmax;
+        int32_t * h_slot = ctx->h_pin, * h_np = h_slot + TM, * hid = h_np + TM, * map = hid + TM * W;
+        for (int t = 0; t < T; ++t) { h_slot[t] = slot; h_np[t] = r0 + t; }
+        std::memcpy(hid, ids + (size_t) r0 * W, (size_t) T * W * 4);
         const int er = spk && spk_pos >= r0 && spk_pos < r0 + T ? spk_pos - r0 : -1;
-        if (er >= 0) for (int k = 0; k < W; ++k) hp_[2 * T + er * W + k] = 0;      // the row's ids are unused
-        int32_t * map = hp_ + 2 * T + T * W;                         // -1 but for the speaker row
-        for (int t = 0; t < T; ++t) map[t] = t == er ? 0 : -1;
-        HIPX(hipMemcpyAsync(ctx->d_slot, hp_, (size_t) T * 4, hipMemcpyHostToDevice, ctx->stream));
-        HIPX(hipMemcpyAsync(ctx->d_npast, hp_ + T, (size_t) T * 4, hipMemcpyHostToDevice, ctx->stream));
-        HIPX(hipMemcpyAsync(ctx->d_ids, hp_ + 2 * T, (size_t) T * W * 4, hipMemcpyHostToDevice, ctx->stream));
         if (er >= 0) {
+            for (int k = 0; k < W; ++k) hid[er * W + k] = 0;                       // the row's ids are unused
+            for (int t = 0; t < T; ++t) map[t] = t == er ? 0 : -1;                 // -1 but for the speaker row
             HIPX(hipMemcpyAsync(ctx->d_emb, sp.data(), (size_t) ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
-            HIPX(hipMemcpyAsync(ctx->d_emb_map, map, (size_t) T * 4, hipMemcpyHostToDevice, ctx->stream));
         }
-        if (int rc = run_step(ctx, T, hp_ + T, ctx->d_slot, ctx->d_npast, ctx->d_ids, er >= 0 ? ctx->d_emb : nullptr,
-                              ctx->logits, /*kv_pre=*/true, er >= 0 ? ctx->d_emb_map : nullptr, hp_, /*f32_prompt=*/true,
+        if (int rc = upload_inputs(ctx, er >= 0 ? (2 + W) * TM + T : 2 * TM + (size_t) T * W)) return rc;
+        if (int rc = run_step(ctx, T, h_np, ctx->d_slot, ctx->d_npast, ctx->d_ids, er >= 0 ? ctx->d_emb : nullptr,
+                              ctx->logits, /*kv_pre=*/true, er >= 0 ? ctx->d_emb_map : nullptr, h_slot, /*f32_prompt=*/true,
                               last ? HEAD_LAST : HEAD_NONE)) return rc;
-        if (last) HIPX(hipMemcpyAsync(last_logits, ctx->logits, row * 4, hipMemcpyDeviceToHost, ctx->stream));
+        if (last) return finish_pass(ctx, last_logits, row);
         HIPX(hipStreamSynchronize(ctx->stream));               // the pinned inputs are reused by the next chunk
     }
-    return check_err_flag(ctx);
+    return Z2H_OK;
 }
 
 int z2h_speaker_embed(z2h_ctx * ctx, int n, const float * spk, const float * delta, float * out) {
@@ -2013,11 +2015,21 @@ int z2h_step_mixed(z2h_ctx * ctx, int n_rows, const int32_t * slot_idx, const in
     if (n_rows <= 0 || n_rows > ctx->Tmax || (ctx->capture && n_rows > ctx->Tstep)) return seterr(ctx, Z2H_EINVAL, "n_rows out of range");
     if (emb_map && (!emb || n_emb <= 0)) return seterr(ctx, Z2H_EINVAL, "emb_map without embedding rows");
     const int W = ctx->W;
-    std::set<std::pair<int, int>> seen;
+    // the cache rows written so far, a bit each; the bits that a call sets are cleared on every way out
+    auto & seen = ctx->row_seen;
+    seen.resize(((size_t) ctx->n_slots * ctx->S + 63) / 64);
+    struct Marks {
+        std::vector<uint64_t> & bits; const int32_t * slot, * pos; size_t S; int n = 0;
+        ~Marks() { for (int t = 0; t < n; ++t) bits[at(t) / 64] = 0; }
+        size_t at(int t) const { return (size_t) slot[t] * S + pos[t]; }
+    } marks{seen, slot_idx, n_past, (size_t) ctx->S};
     for (int t = 0; t < n_rows; ++t) {
         if (slot_idx[t] < 0 || slot_idx[t] >= ctx->n_slots) return seterr(ctx, Z2H_EINVAL, "slot index out of range");
         if (n_past[t] < 0 || n_past[t] >= ctx->S) return seterr(ctx, Z2H_EINVAL, "n_past out of range");
-        if (!seen.insert({slot_idx[t], n_past[t]}).second) return seterr(ctx, Z2H_EINVAL, "two rows write the same cache row");
+        const size_t cr = marks.at(t);
+        if (seen[cr / 64] >> (cr % 64) & 1) return seterr(ctx, Z2H_EINVAL, "two rows write the same cache row");
+        seen[cr / 64] |= (uint64_t) 1 << (cr % 64);
+        marks.n = t + 1;
         const int em = emb_map ? emb_map[t] : -1;
         if (em < -1 || em >= n_emb) return seterr(ctx, Z2H_EINVAL, "emb_map entry out of range");
         if (em < 0)
@@ -2032,36 +2044,24 @@ int z2h_step_mixed(z2h_ctx * ctx, int n_rows, const int32_t * slot_idx, const in
     if (emb_map && (size_t) n_emb * ctx->hp.n_embd > (size_t) ctx->Tmax * ctx->hp.n_embd) return seterr(ctx, Z2H_EINVAL, "too many embedding rows");
     HIPX(hipSetDevice(ctx->device));
     ctx->resident_T = ctx->resident_last = 0;
-    int32_t * hp_ = ctx->h_pin;
-    std::memcpy(hp_, slot_idx, (size_t) n_rows * 4);
-    std::memcpy(hp_ + n_rows, n_past, (size_t) n_rows * 4);
-    int32_t * hid = hp_ + 2 * n_rows;
+    const size_t TM = ctx->Tmax;
+    int32_t * h_slot = ctx->h_pin, * h_np = h_slot + TM, * hid = h_np + TM, * map = hid + TM * W, * hrows = map + TM;
+    std::memcpy(h_slot, slot_idx, (size_t) n_rows * 4);
+    std::memcpy(h_np, n_past, (size_t) n_rows * 4);
     std::memcpy(hid, ids, (size_t) n_rows * W * 4);
-    int32_t * map = hid + (size_t) n_rows * W;
-    for (int t = 0; t < n_rows; ++t) {
-        map[t] = emb_map ? emb_map[t] : -1;
+    for (int t = 0; emb_map && t < n_rows; ++t) {
+        map[t] = emb_map[t];
         if (map[t] >= 0) for (int k = 0; k < W; ++k) hid[(size_t) t * W + k] = 0;     // unused ids
     }
-    HIPX(hipMemcpyAsync(ctx->d_slot, hp_, (size_t) n_rows * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPX(hipMemcpyAsync(ctx->d_npast, hp_ + n_rows, (size_t) n_rows * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPX(hipMemcpyAsync(ctx->d_ids, hid, (size_t) n_rows * W * 4, hipMemcpyHostToDevice, ctx->stream));
-    if (emb_map) {
-        HIPX(hipMemcpyAsync(ctx->d_emb_map, map, (size_t) n_rows * 4, hipMemcpyHostToDevice, ctx->stream));
-        HIPX(hipMemcpyAsync(ctx->d_emb, emb, (size_t) n_emb * ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
-    }
-    // the requested rows' indices (pinned, after the ids and the embedding map)
-    int32_t * hrows = map + n_rows;
-    std::memcpy(hrows, out_rows, (size_t) n_out * 4);
-    if (n_out > 0) HIPX(hipMemcpyAsync(ctx->d_head_rows, hrows, (size_t) n_out * 4, hipMemcpyHostToDevice, ctx->stream));
+    if (n_out > 0) std::memcpy(hrows, out_rows, (size_t) n_out * 4);
+    if (int rc = upload_inputs(ctx, n_out > 0 ? (3 + W) * TM + n_out : emb_map ? (2 + W) * TM + n_rows : 2 * TM + (size_t) n_rows * W)) return rc;
+    if (emb_map) HIPX(hipMemcpyAsync(ctx->d_emb, emb, (size_t) n_emb * ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
     // every row appends its K/V before the attention; a slot's rows attend causally to each other; the
     // head runs on the requested rows only
-    if (int rc = run_step(ctx, n_rows, hp_ + n_rows, ctx->d_slot, ctx->d_npast, ctx->d_ids, emb_map ? ctx->d_emb : nullptr,
-                          ctx->logits, /*kv_pre=*/true, emb_map ? ctx->d_emb_map : nullptr, hp_, false,
+    if (int rc = run_step(ctx, n_rows, h_np, ctx->d_slot, ctx->d_npast, ctx->d_ids, emb_map ? ctx->d_emb : nullptr,
+                          ctx->logits, /*kv_pre=*/true, emb_map ? ctx->d_emb_map : nullptr, h_slot, false,
                           HEAD_ROWS, ctx->d_head_rows, n_out)) return rc;
-    const size_t row = (size_t) ctx->hp.n_codebooks * ctx->hp.audio_vocab;
-    if (n_out > 0) HIPX(hipMemcpyAsync(out_logits, ctx->logits, (size_t) n_out * row * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    return check_err_flag(ctx);
+    return finish_pass(ctx, out_logits, (size_t) n_out * ctx->hp.n_codebooks * ctx->hp.audio_vocab);
 }
 
 int z2h_set_prefill_chunk(z2h_ctx * ctx, int rows) {
