@@ -686,9 +686,15 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
         }
 #undef GQ
     } else {
-        // wide tiles (64 token rows) for wide dense passes and experts averaging 32+ routes, else
-        // narrow ones (16 token rows, 16 output rows per wave)
+        // wide tiles (64 token rows) for wide dense passes and experts averaging 32+ routes; narrower dense
+        // passes k_gemm_f16_few (64 rows, where its lead ends: 39 us against 35); narrower experts and
+        // the dense SwiGLU narrow tiles (16 token rows, 16 output rows per wave)
         const bool wide = a.grouped ? a.n_tok * a.k >= 32 * a.E : a.n_tok >= GEMM_MIN_ROWS;
+        if (!wide && !a.grouped && !dual && a.epi != EPI_ROUTE_W) {
+            KL(k_gemm_f16_few, dim3((m0.rows + 15) / 16, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);
+            HIPX(hipGetLastError());
+            return Z2H_OK;
+        }
         const int rpb = wide ? (dual ? 128 : 256) : 64;
         const dim3 grid((m0.rows + rpb - 1) / rpb, gemm_slots(a.grouped, a.n_tok, a.k, a.E, wide ? 64 : 16));
         const size_t lds = gemm_f16_lds(wide ? 4 : 1);
