@@ -70,38 +70,44 @@ __device__ __forceinline__ bool fa_locate(const int32_t * n_past, const int32_t 
     return found;
 }
 
-// The block's output rows [m][GRP * HD] in s_out: stored to o_out (the group's slice of each row) and
-// encoded for W_o (Q8_K per 256-block by one wave, as encode_row; Q8_0 / F16 through encode_row).
-template <int HD, int GRP>
+// The block's output rows [m][GRP * HD] in s_out: encoded for W_o a 256-block per wave (encode_row's
+// arithmetic, four elements per lane, all NW waves of the block; the host encodes in the block only when the span
+// covers whole 256-blocks), and stored to o_out (the group's slice of each row) where something reads them there: a
+// separate encoder, or a capture. 16 rows of 512: 8 to 18 thousand cycles for Q8_K and Q8_0 by four waves, a row
+// at a time. With it and the branch-free queries, 333 rows of a prompt (16 query heads, Q8_0): 27.7 -> 20.8 us, 77 (Q8_K)
+// 16.8 -> 14.1, 1024 48.5 -> 45.2; a mixed pass of 2088 rows (F16) 57 -> 50.
+template <int HD, int GRP, int NW>
 __device__ __forceinline__ void fa_store_rows(const AttnArgs & a, const float * s_out, int t0, int m, int g) {
-    constexpr int SPAN = GRP * HD;
+    constexpr int SPAN = GRP * HD, NB = SPAN / 256 > 0 ? SPAN / 256 : 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int base = g * SPAN, W = a.nh * HD;
-    for (int i = tid; i < m * (SPAN / 4); i += 256) {
-        const int r = i / (SPAN / 4), c = 4 * (i % (SPAN / 4));
-        *(float4 *) (a.o_out + (int64_t) (t0 + r) * W + base + c) = *(const float4 *) (s_out + r * SPAN + c);
-    }
+    if (a.act_fmt == ACT_NONE || a.cap_gate)
+        for (int i = tid; i < m * (SPAN / 4); i += 64 * NW) {
+            const int r = i / (SPAN / 4), c = 4 * (i % (SPAN / 4));
+            *(float4 *) (a.o_out + (int64_t) (t0 + r) * W + base + c) = *(const float4 *) (s_out + r * SPAN + c);
+        }
     if (a.act_fmt == ACT_NONE) return;
     const int Kp = kpad(W);
-    if (a.act_fmt == ACT_Q8_K) {
-        // (the host encodes in the block only when the span covers whole 256-blocks)
-        constexpr int NB = SPAN / 256 > 0 ? SPAN / 256 : 1;
-        for (int b = wave; b < m * (SPAN / 256); b += 4) {
-            const int r = b / NB, bb = b % NB, t = t0 + r;
-            const float4 v4 = *(const float4 *) (s_out + r * SPAN + 256 * bb + 4 * lane);
-            const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-            q8k_block_v(v, a.act.q + (int64_t) t * Kp + base + 256 * bb, a.act.d256 + (int64_t) t * (Kp / 256) + base / 256 + bb,
-                        a.act.bs + (int64_t) t * (Kp / 16) + base / 16 + 16 * bb, lane);
+#pragma unroll 2
+    for (int b = wave; b < m * (SPAN / 256); b += NW) {
+        const int r = b / NB, at = base + 256 * (b % NB), t = t0 + r;
+        const float4 v4 = *(const float4 *) (s_out + r * SPAN + 256 * (b % NB) + 4 * lane);
+        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+        int8_t * q = a.act.q + (int64_t) t * Kp + at;
+        if (a.act_fmt == ACT_Q8_K) {
+            q8k_block_v(v, q, a.act.d256 + (int64_t) t * (Kp / 256) + at / 256, a.act.bs + (int64_t) t * (Kp / 16) + at / 16, lane);
+        } else if (a.act_fmt == ACT_Q8_0) {
+            const float mx = max8_f(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+            const float dd = mx / 127.0f, id = mx != 0.0f ? 127.0f / mx : 0.0f;
+            uint32_t w = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w |= ((uint32_t) (int) rintf(v[i] * id) & 255u) << (8 * i);
+            *(uint32_t *) (q + 4 * lane) = w;
+            if ((lane & 7) == 0) a.act.d32[(int64_t) t * (Kp / 32) + at / 32 + (lane >> 3)] = h2f(f2h(dd));
+        } else {
+            *(uint2 *) (a.act.h + (int64_t) t * Kp + at + 4 * lane) =
+                make_uint2((uint32_t) f2h(v[0]) | ((uint32_t) f2h(v[1]) << 16), (uint32_t) f2h(v[2]) | ((uint32_t) f2h(v[3]) << 16));
         }
-        return;
-    }
-    for (int r = 0; r < m; ++r) {
-        const int t = t0 + r;
-        if (a.act_fmt == ACT_Q8_0)
-            encode_row<ACT_Q8_0>(s_out + r * SPAN, SPAN, a.act.q + (int64_t) t * Kp + base, a.act.d32 + (int64_t) t * (Kp / 32) + base / 32,
-                                 nullptr, nullptr, nullptr);
-        else
-            encode_row<ACT_F16>(s_out + r * SPAN, SPAN, nullptr, nullptr, nullptr, nullptr, a.act.h + (int64_t) t * Kp + base);
     }
 }
 
@@ -352,7 +358,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_fa(AttnArgs a) {
         if (m1 > 0) {
             if (a.cap_gate && rh_ok && fin && q4 == 0 && split == 0) a.cap_gate[(int64_t) t_row * a.nh + qh] = gsig;
             lds_sync();                                               // s_out rows complete
-            fa_store_rows<HD, GRP>(a, s_out, t0, m1, g);
+            fa_store_rows<HD, GRP, 4>(a, s_out, t0, m1, g);
         }
         lds_sync();                                                   // LDS reuse by the next item
     }
@@ -423,7 +429,7 @@ __global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
         *(float4 *) (s_out + h * HD + d4) = make_float4(o.x * f, o.y * f, o.z * f, o.w * f);
     }
     lds_sync();
-    fa_store_rows<HD, GRP>(a, s_out, t, 1, g);
+    fa_store_rows<HD, GRP, 4>(a, s_out, t, 1, g);
 }
 
 // ------------------------------------------------------------------ wide passes, one flash pass per tile
@@ -480,12 +486,10 @@ constexpr float FL_TAU = 8.0f;                                       // lazy res
 
 template <int GRP>
 __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
-    constexpr int HD = 128, NP = HD / 2, DT = HD / 16, KS = HD / 32, RW = HD / 8;   // RW: uint4 per row
+    constexpr int HD = 128, DT = HD / 16, KS = HD / 32, RW = HD / 8;   // RW: uint4 per row
     static_assert(GRP <= 4, "at most 64 row-heads per tile");
     extern __shared__ __attribute__((aligned(16))) char sm_fh[];
     float * s_q = (float *) sm_fh;                                   // [64][HD + 4] queries (before the loop)
-    float2 * s_cs = (float2 *) (sm_fh + 64 * (HD + 4) * 4);          // [16][NP] RoPE (cos, sin)
-    float * s_th = (float *) (sm_fh + 64 * (HD + 4) * 4 + 16 * NP * 8);   // [16][NP] RoPE angles
     float * s_mrg = (float *) sm_fh;                                 // [4][34][64] key-half partials (after)
     float * s_out = (float *) (sm_fh + 4 * 34 * 64 * 4);             // [16][GRP * HD] output rows (after)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q4 = lane >> 4, c16 = lane & 15;
@@ -527,47 +531,36 @@ __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
         }                                                                                                   \
     }
     FH_LOAD(0)
-    // ---- RoPE angle chains (one thread per row), (cos, sin) per (row, dim pair), then the queries
-    // (wave w: row-heads w, w + 8, ...; per-head RMSNorm, |temp|, RoPE; f16 for the products)
-    if (tid < m) {
-        float th = (float) (p0 + tid);
-        for (int j = 0; j < NP; ++j) {
-            s_th[tid * NP + j] = th;
-            th = th * a.theta_scale;
-        }
-    }
-    lds_sync();
-    for (int i = tid; i < m * NP; i += 512) {
-        float sn, cs;
-        z_sincos(s_th[i], sn, cs);
-        s_cs[i] = make_float2(cs, sn);
-    }
-    lds_sync();
+    // ---- queries (wave w: row-heads w, w + 8, ...; per-head RMSNorm, |temp|, RoPE; f16 for the products)
     {
+        // every input (the RoPE pairs from the per-position table) is loaded before the arithmetic, and all row-heads
+        // are formed without branches, so that their reductions overlap (row-heads past P repeat the last)
         constexpr int QW = 8;
-        float2 xq[QW];
+        float2 xq[QW], cq[QW];
+        float mul[QW];
 #pragma unroll
         for (int k = 0; k < QW; ++k) {
             const int rq = min(wave + 8 * k, P - 1), i = rq / GRP, qh = g * GRP + rq % GRP;
             xq[k] = *(const float2 *) (a.qkvg + (int64_t) (t0 + i) * a.R + (int64_t) qh * HD + 2 * lane);
+            rope_at(a, p0 + i, lane, cq[k].x, cq[k].y);
+            mul[k] = a.temp[qh];
         }
+        float2 y[QW];
+#pragma unroll
+        for (int k = 0; k < QW; ++k) norm_rope<HD>(xq[k].x, xq[k].y, mul[k], a.qk_eps, cq[k].x, cq[k].y, y[k].x, y[k].y);
 #pragma unroll
         for (int k = 0; k < QW; ++k) {
             const int rq = wave + 8 * k;
-            if (rq < P) {                                            // (wave-uniform)
-                const int i = rq / GRP, qh = g * GRP + rq % GRP;
-                const float2 c = s_cs[i * NP + lane];
-                float y0, y1;
-                norm_rope<HD>(xq[k].x, xq[k].y, a.temp[qh], a.qk_eps, c.x, c.y, y0, y1);
-                *(float2 *) &s_q[rq * (HD + 4) + 2 * lane] = make_float2(y0, y1);
-                if (a.cap_q) *(float2 *) (a.cap_q + ((int64_t) (t0 + i) * a.nh + qh) * HD + 2 * lane) = make_float2(y0, y1);
-            }
+            if (rq >= P) continue;                                   // (wave-uniform)
+            *(float2 *) &s_q[rq * (HD + 4) + 2 * lane] = y[k];
+            if (a.cap_q) *(float2 *) (a.cap_q + ((int64_t) (t0 + rq / GRP) * a.nh + g * GRP + rq % GRP) * HD + 2 * lane) = y[k];
         }
     }
     lds_sync();
     const int rh = 16 * wq + c16;                                    // the lane's row-head (B columns)
     const bool rh_ok = rh < P;
     const int row = rh_ok ? rh / GRP : 0, pos = p0 + row;
+    const float gate_x = a.qkvg[(int64_t) (t0 + row) * a.R + (int64_t) (a.nh + 2 * nkv) * HD + g * GRP + rh % GRP];   // (ahead of its use)
     // f16(Q[rh][32 ks + 8 q4 .. + 7]) (the f16 query of the K / V products); the scores are taken to
     // log2 units in fp32 (times scale * log2(e)), so P = exp2(S - m)
     const float qscale = a.scale * 1.44269504088896341f;
@@ -666,7 +659,7 @@ __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
         const float a0 = __builtin_amdgcn_exp2f(m_run - M), a1 = __builtin_amdgcn_exp2f(m1 - M);
         const float l = __builtin_fmaf(l_run, a0, l1 * a1);
         const int h = rh % GRP, qhd = g * GRP + h, t = t0 + row;
-        const float gsig = z_sigmoid(a.qkvg[(int64_t) t * a.R + (int64_t) (a.nh + 2 * nkv) * HD + qhd]);
+        const float gsig = z_sigmoid(gate_x);
         const float f = gsig / l;
         if (a.cap_gate && q4 == 0) a.cap_gate[(int64_t) t * a.nh + qhd] = gsig;
 #pragma unroll
@@ -678,7 +671,7 @@ __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
         }
     }
     lds_sync();
-    if (wave < 4) fa_store_rows<HD, GRP>(a, s_out, t0, m, g);        // (a 256-thread helper)
+    fa_store_rows<HD, GRP, 8>(a, s_out, t0, m, g);
 #undef FH_LOAD
 #undef FH_STORE
 }
@@ -712,12 +705,10 @@ __host__ __device__ inline size_t attn_flash32_lds() { return (size_t) 2 * FL_BU
 
 template <int GRP>
 __global__ void __launch_bounds__(512) k_attn_flash32(AttnArgs a) {
-    constexpr int HD = 128, NP = HD / 2, DT = HD / 16, KS = HD / 32, RW = HD / 8;   // RW: 16-byte chunks per plane row
+    constexpr int HD = 128, DT = HD / 16, KS = HD / 32, RW = HD / 8;   // RW: 16-byte chunks per plane row
     static_assert(GRP <= 4, "at most 64 row-heads per tile");
     extern __shared__ __attribute__((aligned(16))) char sm_fl[];
     float * s_q = (float *) sm_fl;                                   // [64][HD + 4] queries (before the loop)
-    float2 * s_cs = (float2 *) (sm_fl + 64 * (HD + 4) * 4);          // [16][NP] RoPE (cos, sin)
-    float * s_th = (float *) (sm_fl + 64 * (HD + 4) * 4 + 16 * NP * 8);   // [16][NP] RoPE angles
     float * s_mrg = (float *) sm_fl;                                 // [4][34][64] key-half partials (after)
     float * s_out = (float *) (sm_fl + 4 * 34 * 64 * 4);             // [16][GRP * HD] output rows (after)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q4 = lane >> 4, c16 = lane & 15;
@@ -768,48 +759,35 @@ __global__ void __launch_bounds__(512) k_attn_flash32(AttnArgs a) {
     }
 #define FL_STORE(B_) FL_STK(B_, 0) FL_STK(B_, 1) FL_STK(B_, 2) FL_STK(B_, 3) FL_STV(B_, 0) FL_STV(B_, 1)
     FL_LOAD(0)
-    // ---- RoPE: each row's angle chain theta_j = pos * theta_scale^j by repeated fp32 multiplication
-    // (one thread per row), then (cos, sin) of every (row, dim pair)
-    if (tid < m) {
-        float th = (float) (p0 + tid);
-        for (int j = 0; j < NP; ++j) {
-            s_th[tid * NP + j] = th;
-            th = th * a.theta_scale;
-        }
-    }
-    lds_sync();
-    for (int i = tid; i < m * NP; i += 512) {
-        float sn, cs;
-        z_sincos(s_th[i], sn, cs);
-        s_cs[i] = make_float2(cs, sn);
-    }
-    lds_sync();
-    // ---- queries: wave w forms row-heads w, w + 8, ... (lane = dim pair): per-head RMSNorm, |temp|,
-    // RoPE; every input load of the wave is issued before the arithmetic
+    // ---- queries: wave w forms row-heads w, w + 8, ... (lane = dim pair): per-head RMSNorm, |temp|, RoPE
     {
-        constexpr int QW = 8;                                        // row-heads per wave at most
-        float2 xq[QW];
+        // every input (the RoPE pairs from the per-position table) is loaded before the arithmetic, and all row-heads
+        // are formed without branches, so that their reductions overlap (row-heads past P repeat the last)
+        constexpr int QW = 8;
+        float2 xq[QW], cq[QW];
+        float mul[QW];
 #pragma unroll
         for (int k = 0; k < QW; ++k) {
             const int rq = min(wave + 8 * k, P - 1), i = rq / GRP, qh = g * GRP + rq % GRP;
             xq[k] = *(const float2 *) (a.qkvg + (int64_t) (t0 + i) * a.R + (int64_t) qh * HD + 2 * lane);
+            rope_at(a, p0 + i, lane, cq[k].x, cq[k].y);
+            mul[k] = a.temp[qh];
         }
+        float2 y[QW];
+#pragma unroll
+        for (int k = 0; k < QW; ++k) norm_rope<HD>(xq[k].x, xq[k].y, mul[k], a.qk_eps, cq[k].x, cq[k].y, y[k].x, y[k].y);
 #pragma unroll
         for (int k = 0; k < QW; ++k) {
             const int rq = wave + 8 * k;
-            if (rq < P) {                                            // (wave-uniform)
-                const int i = rq / GRP, qh = g * GRP + rq % GRP;
-                const float2 c = s_cs[i * NP + lane];
-                float y0, y1;
-                norm_rope<HD>(xq[k].x, xq[k].y, a.temp[qh], a.qk_eps, c.x, c.y, y0, y1);
-                *(float2 *) &s_q[rq * (HD + 4) + 2 * lane] = make_float2(y0, y1);
-            }
+            if (rq >= P) continue;                                   // (wave-uniform)
+            *(float2 *) &s_q[rq * (HD + 4) + 2 * lane] = y[k];
         }
     }
     lds_sync();
     const int rh = 16 * wq + c16;                                    // the lane's row-head (B columns)
     const bool rh_ok = rh < P;
     const int row = rh_ok ? rh / GRP : 0, pos = p0 + row;
+    const float gate_x = a.qkvg[(int64_t) (t0 + row) * a.R + (int64_t) (a.nh + 2 * nkv) * HD + g * GRP + rh % GRP];   // (ahead of its use)
     const float qscale = a.scale * 1.44269504088896341f;             // scores to log2 units
     v8h_t qh[KS], ql[KS];                                            // Q[rh][32 ks + 8 q4 .. + 7] hi / lo
 #pragma unroll
@@ -919,7 +897,7 @@ __global__ void __launch_bounds__(512) k_attn_flash32(AttnArgs a) {
         const float a0 = __builtin_amdgcn_exp2f(m_run - M), a1 = __builtin_amdgcn_exp2f(m1 - M);
         const float l = __builtin_fmaf(l_run, a0, l1 * a1);
         const int h = rh % GRP, qhd = g * GRP + h, t = t0 + row;
-        const float gsig = z_sigmoid(a.qkvg[(int64_t) t * a.R + (int64_t) (a.nh + 2 * nkv) * HD + qhd]);
+        const float gsig = z_sigmoid(gate_x);
         const float f = gsig / l;
         if (a.cap_gate && q4 == 0) a.cap_gate[(int64_t) t * a.nh + qhd] = gsig;
 #pragma unroll
@@ -931,7 +909,7 @@ __global__ void __launch_bounds__(512) k_attn_flash32(AttnArgs a) {
         }
     }
     lds_sync();
-    if (wave < 4) fa_store_rows<HD, GRP>(a, s_out, t0, m, g);        // (a 256-thread helper)
+    fa_store_rows<HD, GRP, 8>(a, s_out, t0, m, g);
 #undef FL_LOAD
 #undef FL_LDK
 #undef FL_LDV
