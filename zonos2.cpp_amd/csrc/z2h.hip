@@ -691,7 +691,9 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
         // the dense SwiGLU narrow tiles (16 token rows, 16 output rows per wave)
         const bool wide = a.grouped ? a.n_tok * a.k >= 32 * a.E : a.n_tok >= GEMM_MIN_ROWS;
         if (!wide && !a.grouped && !dual && a.epi != EPI_ROUTE_W) {
-            KL(k_gemm_f16_few, dim3((m0.rows + 15) / 16, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);
+            // 32 rows per block where more than one wave has tokens and every compute unit keeps a block
+            if (a.n_tok > 16 && m0.rows >= 32 * ctx->n_cu) KL(k_gemm_f16_few<2>, dim3((m0.rows + 31) / 32, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);
+            else KL(k_gemm_f16_few<1>, dim3((m0.rows + 15) / 16, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);
             HIPX(hipGetLastError());
             return Z2H_OK;
         }

@@ -477,40 +477,49 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f16(GemmArgs a) {
         }
 }
 
-// Dense F16 matmuls of few rows (decode widths, the output head): a block owns 16 weight rows and up to 64
+// Dense F16 matmuls of few rows (decode widths, the output head): a block owns 16 G weight rows and up to 64
 // token rows, 16 per wave. Bounded by HBM latency and bytes in flight: one wave streaming its 16 rows (the narrow
 // k_gemm_f16: 145 blocks for the 9225-row head) keeps 8 KB in flight; here the block's 256 threads request
 // the rows' whole K range, in phases of 1024 columns through LDS with two phases in registers, so that 2048
 // columns are in flight at once from every block. Each wave then runs k_gemm_f16's chain of 32-column
-// products for its tokens: same bits. Head of 9225 x 2048: one row 20.7 -> 11.1 us (cold 34 -> 13), 40 rows 37 -> 26, 64 rows 39 -> 35.
-#ifndef Z2H_TEMPLATES_ONLY
+// products for its tokens: same bits. Head of 9225 x 2048, G = 1: one row 20.7 -> 11.1 us (cold 34 -> 13), 40 rows
+// 37 -> 26, 64 rows 39 -> 35. More rows are bounded by the reads of the token rows, 256 KB per block, from L2;
+// G = 2 halves them: 40 rows 23, 64 rows 29.
 constexpr int FEW_SB = 4;                // superblocks per phase
-constexpr int FEW_LD = FEW_SB * 2;       // 16-byte items per thread and phase: 32 FEW_SB chunks x 16 rows
+constexpr int FEW_LD = FEW_SB * 2;       // 16-byte items per thread, phase and group: 32 FEW_SB chunks x 16 rows
+template <int G>
 __global__ void __launch_bounds__(256) k_gemm_f16_few(GemmArgs a) {
-    __shared__ __attribute__((aligned(16))) u32x4 s_w[FEW_SB * 32 * 16];   // [chunk][row]
+    __shared__ __attribute__((aligned(16))) u32x4 s_w[G][FEW_SB * 32 * 16];   // [group][chunk][row]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, K = a.nsb * 256;
-    const int r0 = 16 * blockIdx.x, t0 = 64 * blockIdx.y + 16 * wave, nt = min(16, a.n_tok - t0);
+    const int r0 = 16 * G * blockIdx.x, t0 = 64 * blockIdx.y + 16 * wave, nt = min(16, a.n_tok - t0);
+    // (64-row weight tiles hold whole groups, so a block's last group exists)
     const u32x4 * w = (const u32x4 *) a.w[0] + (size_t) (r0 / 64) * a.nsb * 32 * 64 + r0 % 64 + (tid & 15);
     const int nch = a.nsb * 32, steps = a.nsb * 8;
-    auto load_w = [&](u32x4 (&v)[FEW_LD], int ph) {                  // (chunks past the row repeat the last)
+    auto load_w = [&](u32x4 (&v)[G * FEW_LD], int ph) {              // (chunks past the row repeat the last)
 #pragma unroll
-        for (int j = 0; j < FEW_LD; ++j) v[j] = w[(size_t) min(ph * FEW_SB * 32 + 16 * j + (tid >> 4), nch - 1) * 64];
+        for (int j = 0; j < FEW_LD; ++j)
+#pragma unroll
+            for (int g = 0; g < G; ++g) v[G * j + g] = w[(size_t) min(ph * FEW_SB * 32 + 16 * j + (tid >> 4), nch - 1) * 64 + 16 * g];
     };
-    auto store_w = [&](const u32x4 (&v)[FEW_LD]) {
+    auto store_w = [&](const u32x4 (&v)[G * FEW_LD]) {
 #pragma unroll
-        for (int j = 0; j < FEW_LD; ++j) s_w[(16 * j + (tid >> 4)) * 16 + (tid & 15)] = v[j];
+        for (int j = 0; j < FEW_LD; ++j)
+#pragma unroll
+            for (int g = 0; g < G; ++g) s_w[g][(16 * j + (tid >> 4)) * 16 + (tid & 15)] = v[G * j + g];
     };
     // the wave's token rows (rows past the last repeat it; a wave without rows only stages)
-    const uint16_t * x = a.act.h + (int64_t) (t0 + min(lane & 15, max(nt, 1) - 1)) * K + 8 * q;
+    const uint16_t * x = a.act.h + (int64_t) (nt > 0 ? t0 + min(lane & 15, nt - 1) : 0) * K + 8 * q;
     constexpr int RING = 8;
-    u32x4 A[RING], v[2][FEW_LD];
+    u32x4 A[RING], v[2][G * FEW_LD];
     load_w(v[0], 0);
     if (nt > 0)
 #pragma unroll
         for (int j = 0; j < RING; ++j) A[j] = *(const u32x4 *) (x + 32 * j);   // (steps >= 8)
     load_w(v[1], 1);
-    v4f_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto phase = [&](u32x4 (&cur)[FEW_LD], int ph) {
+    v4f_t acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = (v4f_t) {0.0f, 0.0f, 0.0f, 0.0f};
+    auto phase = [&](u32x4 (&cur)[G * FEW_LD], int ph) {
         if (ph) lds_sync();                                          // the last phase is read
         store_w(cur);
         load_w(cur, ph + 2);
@@ -521,8 +530,11 @@ __global__ void __launch_bounds__(256) k_gemm_f16_few(GemmArgs a) {
             const int k0 = (ph * FEW_SB + sb) * 8;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const v8h_t B = __builtin_bit_cast(v8h_t, s_w[(4 * (sb * 8 + j) + q) * 16 + (lane & 15)]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h_t, A[j]), B, acc, 0, 0, 0);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const v8h_t B = __builtin_bit_cast(v8h_t, s_w[g][(4 * (sb * 8 + j) + q) * 16 + (lane & 15)]);
+                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h_t, A[j]), B, acc[g], 0, 0, 0);
+                }
                 A[j] = *(const u32x4 *) (x + 32 * min(k0 + j + RING, steps - 1));
             }
         }
@@ -531,11 +543,13 @@ __global__ void __launch_bounds__(256) k_gemm_f16_few(GemmArgs a) {
         phase(v[0], ph);
         if ((ph + 1) * FEW_SB < a.nsb) phase(v[1], ph + 1);
     }
-    const int row = r0 + (lane & 15);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (4 * q + i < nt && row < a.rows) a.out[(int64_t) (t0 + 4 * q + i) * a.out_ld + row] = gemm_epi(a, acc[i], 0.0f);
+    for (int g = 0; g < G; ++g) {
+        const int row = r0 + 16 * g + (lane & 15);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < nt && row < a.rows) a.out[(int64_t) (t0 + 4 * q + i) * a.out_ld + row] = gemm_epi(a, acc[g][i], 0.0f);
+    }
 }
-#endif
 
 } // namespace z2d
