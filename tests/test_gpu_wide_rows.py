@@ -1,7 +1,8 @@
-"""Wide MoE layer calls (more than 64 rows: k_router_down_t, and k_gemm_q4k for Q4_K experts) against calls
+"""Wide MoE layer calls (more than 64 rows: k_router_down_t, k_gemm_q4k for Q4_K experts, k_gemm_f16's
+64- and 128-row tiles for F16 ones) against calls
 of at most 16 rows of the same layer: same bits. Model widths that fill and do not fill the router's 64
 chains per step, and more than 2048 columns (two halves); rows that leave remainders in the router's
-4-token tiles and its grid, and in the GEMM's 32- and 64-row tiles."""
+4-token tiles and its grid, and in the GEMMs' tiles."""
 import numpy as np
 import pytest
 
@@ -13,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("bulk,d,E,k,ff,T", [
     (configs.Q8_0, 320, 4, 2, 256, 65), (configs.Q8_0, 2080, 4, 1, 256, 67), (configs.Q8_0, 4096, 2, 1, 256, 70),
-    (configs.F16, 2048, 4, 2, 256, 2051), (configs.Q4_K, 256, 2, 1, 256, 65), (configs.Q4_K, 512, 4, 2, 768, 129),
+    (configs.F16, 2048, 4, 2, 256, 2051), (configs.F16, 512, 4, 2, 256, 190), (configs.F16, 768, 4, 2, 512, 300), (configs.Q4_K, 256, 2, 1, 256, 65), (configs.Q4_K, 512, 4, 2, 768, 129),
     (configs.Q4_K, 1024, 2, 2, 1536, 97), (configs.Q4_K, 768, 3, 1, 256, 1300)],
     ids=lambda v: str(v))
 def test_wide_rows_equal_narrow(bulk, d, E, k, ff, T):

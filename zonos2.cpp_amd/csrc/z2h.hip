@@ -698,9 +698,19 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
             return Z2H_OK;
         }
         const int rpb = wide ? (dual ? 128 : 256) : 64;
-        const dim3 grid((m0.rows + rpb - 1) / rpb, gemm_slots(a.grouped, a.n_tok, a.k, a.E, wide ? 64 : 16));
-        const size_t lds = gemm_f16_lds(wide ? 4 : 1);
-        if (wide) {
+        // tiles of 128 rows read the weights half as often, but an expert a few rows past a multiple of 128 costs a
+        // nearly empty tile, and few tiles leave compute units idle. 32 experts of 2048 x 1536, gate/up, us
+        // with 64 and with 128 rows by routes per expert: 75: 141 / 114, 97: 143 / 119, 128: 146 / 178, 188: 194 /
+        // 198, 261: 240 / 196; down: 75: 65 / 79, 97: 86 / 84, 128: 107 / 88, 188: 114 / 96, 261: 152 / 153. Dense
+        // passes have too few tiles (2088 rows: QKV 59 / 75, W_o 57 / 82).
+        const int per = a.grouped ? a.n_tok * a.k / a.E : 0;
+        const bool tall = dual ? (per >= 72 && per < 112) || per >= 224 : per >= 112 && per < 224;
+        const dim3 grid((m0.rows + rpb - 1) / rpb, gemm_slots(a.grouped, a.n_tok, a.k, a.E, tall ? 128 : wide ? 64 : 16));
+        const size_t lds = gemm_f16_lds(tall ? 8 : wide ? 4 : 1);
+        if (tall) {
+            if (dual) KL((k_gemm_f16<true, 4, 8>), grid, dim3(256), lds, ctx->stream, a);
+            else KL((k_gemm_f16<false, 4, 8>), grid, dim3(256), lds, ctx->stream, a);
+        } else if (wide) {
             if (dual) KL((k_gemm_f16<true, 4, 4>), grid, dim3(256), lds, ctx->stream, a);
             else KL((k_gemm_f16<false, 4, 4>), grid, dim3(256), lds, ctx->stream, a);
         } else {
@@ -1394,6 +1404,7 @@ int set_lds_limits(std::string & err) {
     LDS_ATTR(k_attn_flash32<1>) LDS_ATTR(k_attn_flash32<2>) LDS_ATTR(k_attn_flash32<4>)
     LDS_ATTR(k_attn_flash16<1>) LDS_ATTR(k_attn_flash16<2>) LDS_ATTR(k_attn_flash16<4>)
     LDS_ATTR((k_gemm_f16<true, 4, 4>)) LDS_ATTR((k_gemm_f16<false, 4, 4>)) LDS_ATTR((k_gemm_f16<true, 2, 1>)) LDS_ATTR((k_gemm_f16<false, 1, 1>))
+    LDS_ATTR((k_gemm_f16<true, 4, 8>)) LDS_ATTR((k_gemm_f16<false, 4, 8>))
 #define LDS_TF(H_) LDS_ATTR((k_attn_tile_f32<H_, 1>)) LDS_ATTR((k_attn_tile_f32<H_, 2>)) LDS_ATTR((k_attn_tile_f32<H_, 4>)) LDS_ATTR((k_attn_tile_f32<H_, 8>)) \
                    LDS_ATTR((k_attn_fa<H_, 1>)) LDS_ATTR((k_attn_fa<H_, 2>)) LDS_ATTR((k_attn_fa<H_, 4>)) LDS_ATTR((k_attn_fa<H_, 8>)) \
                    LDS_ATTR((k_attn_merge<H_, 1>)) LDS_ATTR((k_attn_merge<H_, 2>)) LDS_ATTR((k_attn_merge<H_, 4>)) LDS_ATTR((k_attn_merge<H_, 8>))

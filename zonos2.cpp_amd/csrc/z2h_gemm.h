@@ -23,7 +23,6 @@
 
 namespace z2d {
 
-constexpr int GM_HP = 256 + 8;           // LDS pitch of a row's f16 superblock (halves)
 
 typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
@@ -353,36 +352,42 @@ __global__ void __launch_bounds__(256, 2) k_gemm_q4k(GemmArgs a) {
 // does not depend on the width of the pass. grid: x = row blocks of 4 waves, y = tile slots; 256
 // threads; dynamic LDS gemm_f16_lds(TS).
 //   NG: 16-row sub-groups per wave (DUAL: NG / 2 of gate, then the same rows of up)
-//   TS: 16-row token tiles per block tile (GT = 16 * TS token rows)
+//   TS: 16-row token tiles per block tile (GT = 16 * TS token rows). The wide shape is bounded by the weight reads of
+//   a compute unit (64 rows per tile: 16 KB per 32-column step of a block, four steps in flight per wave); TS = 8
+//   halves them per product, its rows staged 128 columns at a time.
+constexpr int gm_f16_steps(int ts) { return ts >= 8 ? 4 : 8; }       // 32-column steps per staged chunk
+constexpr int gm_f16_hp(int ts) { return 32 * gm_f16_steps(ts) + 8; } // LDS pitch of a row's chunk (halves)
 template <int TS>
-struct GmF16 { u32x4 v[TS]; };                                       // half of one superblock's staging
+struct GmF16 { u32x4 v[TS * gm_f16_steps(TS) / 8]; };                // half of one chunk's staging
 
-// half h of one superblock of GT = 16 TS f16 activation rows: GT * 32 16-byte items, 256 TS per half
+// half h of chunk c of GT = 16 TS f16 activation rows
 template <int TS>
-__device__ __forceinline__ void gm_load_f16(GmF16<TS> & st, const ActBuf & act, int K, int sb, int h, const int * s_row) {
+__device__ __forceinline__ void gm_load_f16(GmF16<TS> & st, const ActBuf & act, int K, int c, int h, const int * s_row) {
+    constexpr int N = TS * gm_f16_steps(TS) / 8, RU = 4 * gm_f16_steps(TS);   // items per thread and half; 16-byte items per row
     const int tid = threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < TS; ++j) {
-        const int i = 256 * TS * h + tid + 256 * j, r = i >> 5, c = i & 31;
-        st.v[j] = *(const u32x4 *) (act.h + (int64_t) s_row[r] * K + sb * 256 + c * 8);
+    for (int j = 0; j < N; ++j) {
+        const int i = 256 * N * h + tid + 256 * j, r = i / RU, u = i % RU;
+        st.v[j] = *(const u32x4 *) (act.h + (int64_t) s_row[r] * K + c * (8 * RU) + u * 8);
     }
 }
 template <int TS>
 __device__ __forceinline__ void gm_store_f16(const GmF16<TS> & st, int h, uint16_t * sh) {
+    constexpr int N = TS * gm_f16_steps(TS) / 8, RU = 4 * gm_f16_steps(TS);
     const int tid = threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < TS; ++j) {
-        const int i = 256 * TS * h + tid + 256 * j, r = i >> 5, c = i & 31;
-        *(u32x4 *) (sh + r * GM_HP + c * 8) = st.v[j];
+    for (int j = 0; j < N; ++j) {
+        const int i = 256 * N * h + tid + 256 * j, r = i / RU, u = i % RU;
+        *(u32x4 *) (sh + r * gm_f16_hp(TS) + u * 8) = st.v[j];
     }
 }
 
-__host__ __device__ inline size_t gemm_f16_lds(int ts) { return 2 * (size_t) (16 * ts) * GM_HP * 2 + 3 * (16 * ts) * 4; }
+__host__ __device__ inline size_t gemm_f16_lds(int ts) { return 2 * (size_t) (16 * ts) * gm_f16_hp(ts) * 2 + 3 * (16 * ts) * 4; }
 
 template <bool DUAL, int NG, int TS>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16(GemmArgs a) {
-    constexpr int GT = 16 * TS, BUF = GT * GM_HP;                     // BUF in halves
-    constexpr int RING = NG >= 4 ? 4 : 8;                            // 32-column weight steps in flight
+    constexpr int CS = gm_f16_steps(TS), HP = gm_f16_hp(TS), GT = 16 * TS, BUF = GT * HP;   // BUF in halves
+    constexpr int RING = TS >= 8 ? 2 : NG >= 4 ? 4 : 8;              // 32-column weight steps in flight
     constexpr int RPW = DUAL ? 8 * NG : 16 * NG;                     // output rows per wave
     extern __shared__ __attribute__((aligned(16))) char smem[];
     uint16_t * sh0 = (uint16_t *) smem;
@@ -426,30 +431,39 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f16(GemmArgs a) {
     for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int ts = 0; ts < TS; ++ts) acc[g][ts] = (v4f_t) {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int sb = 0; sb < a.nsb; ++sb) {
-        // the next superblock's rows go into the other buffer (free: every wave passed the barrier
+    const int nch = nsteps / CS;
+    const bool tall = __builtin_amdgcn_readfirstlane(nt) > GT / 2;   // (TS 8: the upper half of the tile has rows)
+    for (int ck = 0; ck < nch; ++ck) {
+        // the next chunk's rows go into the other buffer (free: every wave passed the barrier
         // after its last reads) in two halves, so only half of them occupy registers at a time
-        const uint16_t * sh = sh0 + (sb & 1) * BUF;
-        uint16_t * nb = sh0 + ((sb + 1) & 1) * BUF;
-        const bool more = sb + 1 < a.nsb;
+        const uint16_t * sh = sh0 + (ck & 1) * BUF;
+        uint16_t * nb = sh0 + ((ck + 1) & 1) * BUF;
+        const bool more = ck + 1 < nch;
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            if (more && kb == 0) gm_load_f16<TS>(st, a.act, K, sb + 1, 0, s_row);
-            if (more && kb == 3) { gm_store_f16<TS>(st, 0, nb); gm_load_f16<TS>(st, a.act, K, sb + 1, 1, s_row); }
-            if (more && kb == 6) gm_store_f16<TS>(st, 1, nb);
+        for (int kb = 0; kb < CS; ++kb) {
+            if (more && kb == 0) gm_load_f16<TS>(st, a.act, K, ck + 1, 0, s_row);
+            if (more && kb == (CS == 4 ? 2 : 3)) { gm_store_f16<TS>(st, 0, nb); gm_load_f16<TS>(st, a.act, K, ck + 1, 1, s_row); }
+            if (more && CS == 8 && kb == 6) gm_store_f16<TS>(st, 1, nb);
             if (has) {
-                const int kk = sb * 8 + kb;
-                u32x4 (&b)[NG] = ring[kb % RING];                    // = kk % RING: RING divides 8
-#pragma unroll
-                for (int ts = 0; ts < TS; ++ts) {
-                    const v8h_t A = *(const v8h_t *) (sh + (ts * 16 + (lane & 15)) * GM_HP + 32 * kb + 8 * q);
+                const int kk = ck * CS + kb;
+                u32x4 (&b)[NG] = ring[kb % RING];                    // = kk % RING: RING divides CS
+                auto mul = [&](int ts) {
+                    const v8h_t A = *(const v8h_t *) (sh + (ts * 16 + (lane & 15)) * HP + 32 * kb + 8 * q);
 #pragma unroll
                     for (int g = 0; g < NG; ++g)
                         acc[g][ts] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, __builtin_bit_cast(v8h_t, b[g]), acc[g][ts], 0, 0, 0);
+                };
+                constexpr int T1 = TS >= 8 ? TS / 2 : TS;
+#pragma unroll
+                for (int ts = 0; ts < T1; ++ts) mul(ts);
+                if (T1 < TS && tall) {
+#pragma unroll
+                    for (int ts = T1; ts < TS; ++ts) mul(ts);
                 }
                 if (kk + RING < nsteps) load_step(kk + RING, b);
             }
         }
+        if (more && CS == 4) gm_store_f16<TS>(st, 1, nb);
         lds_sync();
     }
     if (!has) return;
