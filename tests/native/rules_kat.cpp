@@ -1,0 +1,14 @@
+// The dispatch rules of z2h_rules.h for one query per line of stdin; prints 0 or 1 per query.
+#include "../../zonos2.cpp_amd/csrc/z2h_rules.h"
+#include <cstdio>
+#include <cstring>
+
+int main() {
+    char what[32];
+    long long a, b, c, d;
+    while (std::scanf("%31s %lld %lld %lld %lld", what, &a, &b, &c, &d) == 5) {
+        if (!std::strcmp(what, "tall")) std::printf("%d\n", (int) z2r::f16_tall_tiles(a, b, (int) c, (int) d));
+        else return 1;
+    }
+    return 0;
+}

@@ -1,0 +1,50 @@
+"""The host rules that choose between two shapes of one kernel (csrc/z2h_rules.h), on the CPU: the choices at sizes
+where both sides were measured on 256 compute units."""
+import subprocess
+
+import pytest
+
+N_CU = 256
+
+
+@pytest.fixture(scope="module")
+def ask(root, tmp_path_factory):
+    exe = tmp_path_factory.mktemp("rules") / "rules_kat"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", str(root / "tests" / "native" / "rules_kat.cpp"), "-o", str(exe)], check=True)
+
+    def run(queries):
+        text = "\n".join(" ".join(map(str, q)) for q in queries)
+        out = subprocess.run([str(exe)], input=text, check=True, capture_output=True, text=True).stdout.split()
+        assert len(out) == len(queries)
+        return [x == "1" for x in out]
+    return run
+
+
+# (experts, routes per expert, FFN width, model width) -> 128-row tiles: gate/up, down
+TALL = [
+    # too few blocks for the chip: 64-row tiles measured 1.2 to 1.8 times as fast
+    ((16, 93, 1536, 2048), (False, False)), ((16, 128, 1536, 2048), (False, False)), ((8, 128, 1536, 2048), (False, False)),
+    ((4, 512, 1536, 2048), (False, False)), ((8, 260, 256, 512), (False, False)), ((8, 150, 4096, 2048), (True, False)),
+    # a round of tall tiles more than the 64-row ones' rounds are worth
+    ((32, 128, 1536, 2048), (False, True)), ((32, 210, 1536, 2048), (False, False)), ((16, 300, 1536, 2048), (False, True)),
+    # uneven loads: no tall tiles at few routes per expert
+    ((32, 75, 1536, 2048), (False, False)),
+    # rounds saved
+    ((16, 192, 1536, 2048), (True, False)), ((32, 260, 1536, 2048), (True, False)), ((32, 450, 1536, 2048), (True, False)),
+    ((128, 512, 2048, 1024), (True, True)),
+]
+
+
+def test_f16_tall_tiles(ask):
+    q, want = [], []
+    for (E, per, ff, d), w in TALL:
+        q += [("tall", -(-ff // 128), per * E, E, N_CU), ("tall", -(-d // 256), per * E, E, N_CU)]
+        want += w
+    assert ask(q) == want
+
+
+def test_f16_tall_tiles_never_without_a_full_chip(ask):
+    """no tall tiles where the 64-row ones fit one round, whatever the loads"""
+    q = [("tall", rb, items, E, N_CU) for rb in (1, 3, 8, 16, 32) for E in (1, 2, 8, 32, 128) for items in (64, 500, 2047, 9001, 40000)
+         if rb * (items / 64 + E) <= 2 * N_CU]
+    assert q and not any(ask(q))

@@ -10,6 +10,7 @@
 #include "z2h.h"
 #include "z2h_kernels.h"
 #include "z2h_gemm_q.h"
+#include "z2h_rules.h"
 #include "z2h_attn.h"
 #include <hip/hip_ext.h>
 #include "z2_formats.h"
@@ -698,13 +699,8 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
             return Z2H_OK;
         }
         const int rpb = wide ? (dual ? 128 : 256) : 64;
-        // tiles of 128 rows read the weights half as often, but an expert a few rows past a multiple of 128 costs a
-        // nearly empty tile, and few tiles leave compute units idle. 32 experts of 2048 x 1536, gate/up, us
-        // with 64 and with 128 rows by routes per expert: 75: 141 / 114, 97: 143 / 119, 128: 146 / 178, 188: 194 /
-        // 198, 261: 240 / 196; down: 75: 65 / 79, 97: 86 / 84, 128: 107 / 88, 188: 114 / 96, 261: 152 / 153. Dense
-        // passes have too few tiles (2088 rows: QKV 59 / 75, W_o 57 / 82).
-        const int per = a.grouped ? a.n_tok * a.k / a.E : 0;
-        const bool tall = dual ? (per >= 72 && per < 112) || per >= 224 : per >= 112 && per < 224;
+        // (dense passes have too few tiles for 128 rows: 2088 rows, QKV 59 us against 75, W_o 57 against 82)
+        const bool tall = wide && a.grouped && z2r::f16_tall_tiles((m0.rows + rpb - 1) / rpb, (int64_t) a.n_tok * a.k, a.E, ctx->n_cu);
         const dim3 grid((m0.rows + rpb - 1) / rpb, gemm_slots(a.grouped, a.n_tok, a.k, a.E, tall ? 128 : wide ? 64 : 16));
         const size_t lds = gemm_f16_lds(tall ? 8 : wide ? 4 : 1);
         if (tall) {
