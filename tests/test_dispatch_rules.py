@@ -48,3 +48,17 @@ def test_f16_tall_tiles_never_without_a_full_chip(ask):
     q = [("tall", rb, items, E, N_CU) for rb in (1, 3, 8, 16, 32) for E in (1, 2, 8, 32, 128) for items in (64, 500, 2047, 9001, 40000)
          if rb * (items / 64 + E) <= 2 * N_CU]
     assert q and not any(ask(q))
+
+
+# (K, rows, tokens) -> k_gemm_f16_few: where the two differed by more than 5%
+FEW = [
+    ((256, 9234, 16), False), ((256, 9234, 64), False), ((256, 18468, 1), False),
+    ((512, 512, 16), True), ((512, 512, 64), False), ((512, 3078, 16), True), ((512, 4104, 64), False), ((512, 9234, 16), False),
+    ((768, 297, 64), True), ((768, 4104, 64), True), ((768, 9234, 1), True), ((768, 18468, 16), False),
+    ((1024, 1028, 64), True), ((1024, 9234, 16), True), ((1024, 18468, 16), False),
+    ((1536, 18468, 1), True), ((2048, 9225, 1), True), ((2048, 3088, 64), True), ((2048, 18468, 33), True), ((2048, 36864, 16), False),
+]
+
+
+def test_f16_few_rows(ask):
+    assert ask([("few", rows, K // 256, T, 0) for (K, rows, T), _ in FEW]) == [w for _, w in FEW]

@@ -1,4 +1,5 @@
-"""Dense F16 matmuls of few rows (k_gemm_f16_few, 16 or 32 weight rows per block) against the wide GEMM: the columns
+"""Dense F16 matmuls of few rows (k_gemm_f16_few, 16 or 32 weight rows per block, or the narrow k_gemm_f16 where K is short) against the
+wide GEMM: the columns
 of a step of T requests (projections and head of T token rows: one wave's remainder, several waves, all
 64) get the bits of the same columns in steps of at most 16 and in one of 70 (k_gemm_f16). Row lengths of one
 superblock, of part of a phase and of more than two phases; head rows that leave remainders, below and above the
@@ -12,7 +13,7 @@ from zonos2_amd.z2h import Context, Model
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("d,vocab", [(256, 33), (768, 1026), (2304, 1026)])
+@pytest.mark.parametrize("d,vocab", [(256, 33), (512, 33), (512, 1026), (768, 1026), (2304, 1026)])
 def test_few_rows_equal_wide_and_narrow(d, vocab):
     cfg = configs.ModelConfig(f"few-{d}-{vocab}", n_layer=1, n_embd=d, n_head=4, n_head_kv=2, head_dim=64, n_expert=0, top_k=0,
                               n_ff=256, bulk=configs.F16, audio_vocab=vocab, expert_used=[0])

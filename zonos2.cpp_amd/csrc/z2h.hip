@@ -616,7 +616,7 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 // ---------------------------------------------------------------- launch helpers
 // Wide matmuls run as GEMMs, narrow ones as the decode GEMVs; both fold a row's blocks in the same order
 // with the same operations, so the lines below are about speed alone.
-//   F16 (t64)    always k_gemm_f16, in its wide or narrow shape (same bits per row either way).
+//   F16 (t64)    always an MFMA GEMM: k_gemm_f16, wide or narrow, or k_gemm_f16_few (the same bits per row from each).
 //   Q4_K (m16)   passes of more than 64 token rows (k_gemm_q4k's tile height).
 //   Q8_0, Q6_K   dense: more 16-row token tiles x row-group quads than half the compute units. Below that the
 //                K-split GEMV's four times as many blocks win (48 rows of QKV, 147 blocks: 8.0 us against 10.5
@@ -688,10 +688,10 @@ int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvA
 #undef GQ
     } else {
         // wide tiles (64 token rows) for wide dense passes and experts averaging 32+ routes; narrower dense
-        // passes k_gemm_f16_few (64 rows, where its lead ends: 39 us against 35); narrower experts and
-        // the dense SwiGLU narrow tiles (16 token rows, 16 output rows per wave)
+        // passes k_gemm_f16_few where K is long for the rows; the others, narrower experts and the dense SwiGLU
+        // narrow tiles (16 token rows, 16 output rows per wave)
         const bool wide = a.grouped ? a.n_tok * a.k >= 32 * a.E : a.n_tok >= GEMM_MIN_ROWS;
-        if (!wide && !a.grouped && !dual && a.epi != EPI_ROUTE_W) {
+        if (!wide && !a.grouped && !dual && a.epi != EPI_ROUTE_W && z2r::f16_few_rows(m0.rows, a.nsb, a.n_tok)) {
             // 32 rows per block where more than one wave has tokens and every compute unit keeps a block
             if (a.n_tok > 16 && m0.rows >= 32 * ctx->n_cu) KL(k_gemm_f16_few<2>, dim3((m0.rows + 31) / 32, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);
             else KL(k_gemm_f16_few<1>, dim3((m0.rows + 15) / 16, (a.n_tok + 63) / 64), dim3(256), 0, ctx->stream, a);

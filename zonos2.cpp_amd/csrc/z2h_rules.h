@@ -24,4 +24,20 @@ inline bool f16_tall_tiles(int64_t row_blocks, int64_t items, int E, int n_cu) {
     return 1.28 + 0.78 * (n128 - 1) < 1.0 + 0.53 * (n64 - 1);
 }
 
+// Dense F16 matmuls of at most 64 token rows: k_gemm_f16_few (16 or 32 weight rows per block, the whole K range requested at
+// once) instead of k_gemm_f16's narrow shape (64 weight rows per block, 256 columns in flight per wave). It wins by
+// the loads in flight, so by K; it loses by reading the token rows from L2 once per 16 rows, so by rows and tokens.
+// Measured in us, narrow / few, at 1, 16 and 64 tokens:
+//   K 256, 1026 rows 4.8 / 4.8, 4.9 / 4.8, 4.9 / 5.1; 9234 rows 4.8 / 4.8, 5.0 / 6.6, 6.3 / 10.5
+//   K 512, 3078 rows 5.0 / 4.8, 5.9 / 4.9, 7.3 / 6.3; 4104 rows 4.9 / 4.8, 5.8 / 4.9, 7.5 / 8.4; 512 rows 4.0 / 3.9,
+//          4.7 / 4.0, 4.7 / 5.3; 9234 rows 4.9 / 5.1, 6.2 / 7.2, 10.8 / 12.0
+//   K 768, 9234 rows 6.1 / 5.4, 7.7 / 8.0, 14.1 / 14.0; 18468 rows 10.0 / 9.1, 11.0 / 13.6, 20.9 / 21.4
+//   K 1024, 9234 rows 10.8 / 5.3, 12.3 / 8.4, 17.2 / 17.0; 18468 rows 12.9 / 10.6, 14.2 / 15.6, 25.7 / 25.4
+//   K 1536, 18468 rows 19.3 / 13.6, 20.2 / 20.2, 35.4 / 32.9
+//   K 2048, 18468 rows 24.4 / 17.0, 25.8 / 22.7, 45.4 / 39.7; 36864 rows 28.0 / 28.9, 30.2 / 39.2, 58.5 / 61.6
+//   nsb: 256-column superblocks of K
+inline bool f16_few_rows(int64_t rows, int nsb, int n_tok) {
+    return nsb >= 2 && rows <= 4096ll * nsb && (nsb > 2 || n_tok <= 32);
+}
+
 } // namespace z2r
