@@ -9,6 +9,7 @@ int main() {
     while (std::scanf("%31s %lld %lld %lld %lld", what, &a, &b, &c, &d) == 5) {
         if (!std::strcmp(what, "tall")) std::printf("%d\n", (int) z2r::f16_tall_tiles(a, b, (int) c, (int) d));
         else if (!std::strcmp(what, "few")) std::printf("%d\n", (int) z2r::f16_few_rows(a, (int) b, (int) c));
+        else if (!std::strcmp(what, "rdown")) std::printf("%d\n", (int) z2r::router_down_reuse((int) a, (int) b, c != 0));
         else return 1;
     }
     return 0;

@@ -62,3 +62,14 @@ FEW = [
 
 def test_f16_few_rows(ask):
     assert ask([("few", rows, K // 256, T, 0) for (K, rows, T), _ in FEW]) == [w for _, w in FEW]
+
+
+# (rows, model width) -> k_router_down_t in an MoE layer call
+RDOWN = [((65, 768), False), ((200, 768), True), ((65, 1024), False), ((160, 1024), True), ((65, 1280), False), ((112, 1280), True),
+         ((64, 2048), False), ((65, 2048), True), ((65, 2304), False), ((72, 3072), False), ((96, 3072), True), ((65, 4096), True),
+         ((64, 512), False), ((65, 512), True), ((256, 256), True)]
+
+
+def test_router_down_reuse(ask):
+    full = lambda d: d % 64 == 0 and d // 64 & (d // 64 - 1) == 0
+    assert ask([("rdown", T, d, int(full(d)), 0) for (T, d), _ in RDOWN]) == [w for _, w in RDOWN]

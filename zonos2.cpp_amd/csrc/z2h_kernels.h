@@ -2376,7 +2376,9 @@ __global__ void __launch_bounds__(256) k_router_down(RouterArgs a) {
 // one's chains run; rows of more than 2048 floats go in two halves, the chains kept in LDS between them.
 // Grid (rd / 16, at most ceil(T / RD_T)), 256 threads, dynamic LDS router_down_t_lds(ni, d).
 // Bounded by the LDS return path (each of a token's 16-byte reads serves 4 fma per lane) and by the rows'
-// first load: d 2048, 128 outputs, 77 rows 16.3 -> 6.3 us, 333 16.9 -> 11.5, 1500 41 -> 34, 2088 50 -> 40.
+// first load. Against a block's 32 outputs over 8 tokens, a wave forming one output at a time: d 2048, 128 outputs, 77 rows
+// 16.3 -> 6.3 us, 333 16.9 -> 11.5, 1500 41 -> 34, 2088 50 -> 40; d 1024, 65 rows 11.2 -> 5.3, 2048 23.5 -> 22.5. It is the slower one
+// at d 4096 from 400 rows (1024: 56 -> 67 us): the halves' weights are read again for every tile.
 constexpr int RD_T = 4;
 __host__ __device__ inline size_t router_down_t_lds(int ni, int d) { return (size_t) RD_T * (4 * d + (ni > 32 ? 4096 : 0)); }
 template <int NI, bool GUARD>

@@ -40,4 +40,16 @@ inline bool f16_few_rows(int64_t rows, int nsb, int n_tok) {
     return nsb >= 2 && rows <= 4096ll * nsb && (nsb > 2 || n_tok <= 32);
 }
 
+// The router down projection alone (an MoE layer call): k_router_down_t, which loads a weight row once for many tokens, instead
+// of k_router_down's block per token and four outputs. Up to 512 columns it is never the slower one; above, it pays from
+// about the work of 65 rows of 2048 columns, and rows of more than 2048 columns that leave part of the last chain step
+// idle (d not 64 times a power of two) from 80 rows. us, per token / reusing,
+// 128 outputs: d 512 at 128 rows 4.2 / 4.2, 256 6.5 / 4.2; d 768 at 65 4.2 / 5.7, 160 6.8 / 7.0, 200 8.0 / 6.5; d 1024 at
+// 65 4.1 / 5.2, 128 6.2 / 5.8; d 1280 at 65 6.2 / 7.9, 96 7.7 / 8.1, 112 8.6 / 8.2; d 2048 at 65 6.6 / 5.4; d 3072
+// at 65 14.4 / 16.0, 80 16.8 / 16.2; d 4096 at 65 10.8 / 8.6.
+//   full: d is 64 times a power of two
+inline bool router_down_reuse(int T, int d, bool full) {
+    return (d <= 512 || (int64_t) T * d >= 65 * 2048) && T >= (d > 2048 && !full ? 80 : 65);
+}
+
 } // namespace z2r
