@@ -4,6 +4,8 @@ GEMVs), at token tiles of every height and their remainders, at rows and K that 
 and with activations whose block scales are f16 subnormals or large. A prompt prefilled in one pass
 (dense projections and dense FFN as GEMMs) gives the bits of 16-row passes. The GEMVs are held to the
 oracle elsewhere; one layer here is too."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -35,6 +37,35 @@ def test_moe_gemm_equals_gemv(bulk, E, k, ff, T, scale):
     got = ctx.moe_forward(0, x)
     want = np.concatenate([ctx.moe_forward(0, x[i:i + 16]) for i in range(0, T, 16)])
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"max |d| {np.abs(got - want).max():.3e}"
+    ctx.close(); m.close()
+
+
+@pytest.mark.parametrize("bulk,offset,f16", [(Q8, 0, 0x7e01), (Q8, 0, 0x7c00), (Q6, 208, 0x7c00)], ids=["q8_0-nan", "q8_0-inf", "q6_k-inf"])
+def test_non_finite_scales_stay_in_their_block(bulk, offset, f16):
+    """a weight block's scale or a token's scale that is infinite or NaN gives what the GEMV gives: the other
+    rows, and the sums of the other blocks, are untouched"""
+    cfg = _cfg(bulk, 2, 2, 512)
+    model = synth.generate_model(cfg, 21)
+    t = model["blk.0.ffn_down_exps.weight"]
+    raw = np.frombuffer(bytes(t.data), np.uint8).copy()
+    rb = configs.row_bytes(bulk, cfg.n_ff)
+    bb = configs.BLOCK[bulk][1]
+    for row, blk in ((5, 1), (37, 0), (cfg.n_embd + 100, 1)):            # experts 0, 0 and 1
+        raw[row * rb + blk * bb + offset:][:2] = np.frombuffer(np.uint16(f16).tobytes(), np.uint8)
+    model["blk.0.ffn_down_exps.weight"] = dataclasses.replace(t, data=raw)
+    m = Model(cfg.hparams(), model)
+    T = 67
+    ctx = Context(None, 1, 256, model=m, max_rows=T)
+    x = np.random.default_rng(2).standard_normal((T, cfg.n_embd)).astype(np.float32)
+    x[3] *= 1e9                                                          # its block scales are infinite in f16
+    print(f"{cfg.name} non-finite scales", flush=True)
+    got = ctx.moe_forward(0, x)
+    want = np.concatenate([ctx.moe_forward(0, x[i:i + 16]) for i in range(0, T, 16)])
+    rest = np.delete(np.arange(cfg.n_embd), [5, 37, 100])
+    assert np.isfinite(want[4:][:, rest]).all() and not np.isfinite(want[:, [5, 37, 100]]).any()
+    if f16 == 0x7c00:
+        assert np.isinf(want[4:][:, [5, 37, 100]]).any()
+    np.testing.assert_array_equal(got, want)                             # (NaN equals NaN)
     ctx.close(); m.close()
 
 

@@ -16,6 +16,7 @@
 #include "z2_formats.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -55,6 +56,7 @@ namespace {
 struct DevMat {
     int type = -1;
     bool m16 = false;                 // 16-row MFMA layout (Q4_K, Q8_0) instead of 64-row tiles
+    bool finite = true;               // Q8_0: no block scale is infinite or NaN (k_gemm_q80 needs that)
     int rows = 0, K = 0, nsb = 0, tiles = 0, n_mats = 1;
     uint8_t * w = nullptr;            // tiled bytes
     uint16_t * dpl = nullptr;         // Q6_K d plane
@@ -281,6 +283,7 @@ int upload_mat_m16(z2h_model * mdl, int type, int64_t K, int64_t rows, int n_mat
     dm.mat_bytes = (int64_t) dm.tiles * dm.nsb * UB;
     const int64_t rb = z2::row_bytes(type, K);
     std::vector<uint8_t> out((size_t) dm.mat_bytes * n_mats, 0);
+    std::atomic<bool> bad{false};                         // a Q8_0 scale with all exponent bits set
     auto do_rows = [&](int64_t g0, int64_t g1) {          // global 16-row group range over all matrices
         for (int64_t gg = g0; gg < g1; ++gg) {
             const int e = (int) (gg / dm.tiles), g = (int) (gg % dm.tiles);
@@ -311,7 +314,9 @@ int upload_mat_m16(z2h_model * mdl, int type, int64_t K, int64_t rows, int n_mat
                     else
                         for (int b = 0; b < 8; ++b) {
                             const int64_t blk = (int64_t) sb * 8 + b;
-                            if (blk * 32 < K) std::memcpy(hd + 2 * b, rp + 34 * blk, 2);
+                            if (blk * 32 >= K) break;
+                            std::memcpy(hd + 2 * b, rp + 34 * blk, 2);
+                            if ((rp[34 * blk + 1] & 0x7c) == 0x7c) bad.store(true, std::memory_order_relaxed);
                         }
                 }
             }
@@ -322,6 +327,7 @@ int upload_mat_m16(z2h_model * mdl, int type, int64_t K, int64_t rows, int n_mat
     std::vector<std::thread> th;
     for (int i = 0; i < nth; ++i) th.emplace_back([&, i] { do_rows(total * i / nth, total * (i + 1) / nth); });
     for (auto & t : th) t.join();
+    dm.finite = !bad;
     if (int rc = dalloc(mdl, &dm.w, out.size(), mdl->bytes_w)) return rc;
     HIPM(hipMemcpy(dm.w, out.data(), out.size(), hipMemcpyHostToDevice));
     return Z2H_OK;
@@ -625,23 +631,24 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 //                27.4). One and two rows keep the token-pair units. Experts: at least 8 routes per expert
 //                on average, where the GEMV starts re-reading its weights per 8- or 16-route pass (64 rows,
 //                top-4 of 32: Q6_K gate/up 38 us against 52, down 22 against 32; 48 rows, 6 routes: level
-//                before the sort launch is counted).
+//                before the sort launch is counted). Q8_0 matrices with an infinite or NaN block scale stay on
+//                the GEMVs at every width: k_gemm_q80 multiplies a row's other scales of the superblock by zero.
 constexpr int GEMM_MIN_ROWS = 65;
 // (k_gemm_q4k's activation offsets are 32-bit)
 bool gemm_q4k_ok(const DevMat & m, int64_t items) { return items * m.nsb * 256 < (int64_t) 1 << 32; }
 bool use_gemm(const z2h_ctx * ctx, const DevMat & m, int n_tok) {
     if (!m.m16) return m.type == Z2H_F16;
     if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, n_tok);
-    return n_tok > 2 && 2ll * ((m.tiles + 3) / 4) * ((n_tok + 15) / 16) > ctx->n_cu;
+    return m.finite && n_tok > 2 && 2ll * ((m.tiles + 3) / 4) * ((n_tok + 15) / 16) > ctx->n_cu;
 }
 bool use_gemm_experts(const DevMat & m, int n_tok, int k, int E) {
     if (!m.m16) return m.type == Z2H_F16;
     if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, (int64_t) n_tok * k);
-    return n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
+    return m.finite && n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
 }
 // gate and up fused with SwiGLU in one GEMM launch: same type, layout and shape
 bool gemm_dual_ok(const DevMat & g, const DevMat & u) {
-    return g.type == u.type && g.m16 == u.m16 && g.nsb == u.nsb && g.tiles == u.tiles && g.rows == u.rows && g.mat_bytes == u.mat_bytes;
+    return g.type == u.type && g.m16 == u.m16 && g.finite == u.finite && g.nsb == u.nsb && g.tiles == u.tiles && g.rows == u.rows && g.mat_bytes == u.mat_bytes;
 }
 
 int launch_gemm(z2h_ctx * ctx, const DevMat & m0, const DevMat * m1, const GemvArgs & g, int fam) {

@@ -11,7 +11,8 @@
 // is scaled and added by itself.
 //   k_gemm_q80   per 32-column block t = t + (dw * dx) * (float) dot, and the 8 blocks' t into the row
 //                sum. dot is an int8 product; dw * dx (f16 x f16, exact in fp32) comes off the vector
-//                unit: it is an f16 product with the token's scales masked to one block, so the
+//                unit: it is an f16 product with the token's scales masked to one block (so the matrix's scales
+//                must be finite; the host sees to that: masking them too took 4% of the kernel), and the
 //                conversion, the multiply by dot and the add stay per output.
 //   k_gemm_q6k   x = (d * dx) * (float) sum_g sc_g * dot_g per superblock. The scale times the 6-bit
 //                value, sc * (w - 32), is formed once per weight and split as 64 * hi + lo (both int8),
