@@ -131,9 +131,10 @@ struct z2h_ctx {
     int Tstep = 0;                    // columns a step may list (n_slots); captures are sized for it
     int pch = 0;                      // prefill chunk rows (<= Tmax)
     int max_rows = 0;                 // requested row capacity (z2h_create_batch_rows)
-    // a pass's integer inputs, one block [(4 + W) Tmax] laid out like h_pin: slot | n_past | ids (W per row) |
-    // per-row embedding override | rows of a mixed pass that get logits
-    int32_t * d_slot = nullptr, * d_npast = nullptr, * d_ids = nullptr, * d_emb_map = nullptr, * d_head_rows = nullptr;
+    // a pass's integer inputs, one block [(4 + W) Tmax] laid out like h_pin. Steps keep slot | n_past | ids (W per
+    // column) at strides of Tstep (captured graphs and z2h_sample_feed hold these addresses); prefill chunks and mixed
+    // passes pack theirs by their own row count (pass_inputs)
+    int32_t * d_slot = nullptr, * d_npast = nullptr, * d_ids = nullptr;
     float * d_emb = nullptr;
     float * spk_io = nullptr;         // speaker projection: spk | lda out | proj out | delta
     float * res = nullptr, * res2 = nullptr, * cur = nullptr, * qkvg = nullptr, * wo_out = nullptr;
@@ -573,7 +574,7 @@ int alloc_scratch(z2h_ctx * ctx) {
     }
     if (hipHostMalloc((void **) &ctx->h_tiles, (size_t) 2 * ctx->items_max * sizeof(int4), hipHostMallocDefault) != hipSuccess)
         return seterr(ctx, Z2H_ENOMEM, "hipHostMalloc failed");
-    ctx->d_npast = ctx->d_slot + T; ctx->d_ids = ctx->d_npast + T; ctx->d_emb_map = ctx->d_ids + (size_t) T * W; ctx->d_head_rows = ctx->d_emb_map + T;
+    ctx->d_npast = ctx->d_slot + ctx->Tstep; ctx->d_ids = ctx->d_npast + ctx->Tstep;
     if (hipHostMalloc((void **) &ctx->h_pin, ((size_t) T * (4 + W) + 4) * 4, hipHostMallocDefault) != hipSuccess)
         return seterr(ctx, Z2H_ENOMEM, "hipHostMalloc failed");
     const int ncb = std::max(1, (int) hp.n_codebooks);
@@ -1487,8 +1488,15 @@ int launch_attn_fa(z2h_ctx * ctx, const AttnArgs & a, int grid) {
     return Z2H_OK;
 }
 
+// The inputs of a pass of T rows within a block (h_pin or d_slot), one after the other: slot | n_past | ids (W per row) |
+// per-row embedding override | rows that get logits (up to Tmax).
+struct PassInputs { int32_t * slot, * n_past, * ids, * emb_map, * head_rows; };
+PassInputs pass_inputs(int32_t * block, size_t T, int W) {
+    return {block, block + T, block + 2 * T, block + (2 + W) * T, block + (3 + W) * T};
+}
+
 // One pinned upload of a pass's integer inputs, the first n ints of h_pin's block. Each copy costs about 8 us of
-// host time and queue time, so a pass makes one.
+// host time and queue time, so a pass makes one; a few rows in a context of 8192 must not send what 8192 would.
 int upload_inputs(z2h_ctx * ctx, size_t n) {
     HIPX(hipMemcpyAsync(ctx->d_slot, ctx->h_pin, n * 4, hipMemcpyHostToDevice, ctx->stream));
     return Z2H_OK;
@@ -1896,11 +1904,11 @@ int z2h_step(z2h_ctx * ctx, int T, const int32_t * slot_idx, const int32_t * n_p
     }
     HIPX(hipSetDevice(ctx->device));
     int32_t * hp_ = ctx->h_pin;
-    const size_t TM = ctx->Tmax;
+    const size_t TS = ctx->Tstep;
     std::memcpy(hp_, slot_idx, (size_t) T * 4);
-    std::memcpy(hp_ + TM, n_past, (size_t) T * 4);
-    if (ids) std::memcpy(hp_ + 2 * TM, ids, (size_t) T * ctx->W * 4);
-    if (int rc = upload_inputs(ctx, ids ? 2 * TM + (size_t) T * ctx->W : TM + T)) return rc;
+    std::memcpy(hp_ + TS, n_past, (size_t) T * 4);
+    if (ids) std::memcpy(hp_ + 2 * TS, ids, (size_t) T * ctx->W * 4);
+    if (int rc = upload_inputs(ctx, ids ? 2 * TS + (size_t) T * ctx->W : TS + T)) return rc;
     if (emb) HIPX(hipMemcpyAsync(ctx->d_emb, emb, (size_t) T * ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
     ctx->resident_T = ctx->resident_last = 0;
     ctx->last_np.assign(n_past, n_past + T);
@@ -2002,19 +2010,18 @@ int z2h_prefill(z2h_ctx * ctx, int slot, const int32_t * ids, int n0, const floa
     for (int r0 = 0; r0 < n0; r0 += chunk) {
         const int T = std::min(chunk, n0 - r0);
         const bool last = r0 + T == n0;
-        const size_t TM = ctx->Tmax;
-        int32_t * h_slot = ctx->h_pin, * h_np = h_slot + TM, * hid = h_np + TM, * map = hid + TM * W;
-        for (int t = 0; t < T; ++t) { h_slot[t] = slot; h_np[t] = r0 + t; }
-        std::memcpy(hid, ids + (size_t) r0 * W, (size_t) T * W * 4);
+        const PassInputs h = pass_inputs(ctx->h_pin, T, W), d = pass_inputs(ctx->d_slot, T, W);
+        for (int t = 0; t < T; ++t) { h.slot[t] = slot; h.n_past[t] = r0 + t; }
+        std::memcpy(h.ids, ids + (size_t) r0 * W, (size_t) T * W * 4);
         const int er = spk && spk_pos >= r0 && spk_pos < r0 + T ? spk_pos - r0 : -1;
         if (er >= 0) {
-            for (int k = 0; k < W; ++k) hid[er * W + k] = 0;                       // the row's ids are unused
-            for (int t = 0; t < T; ++t) map[t] = t == er ? 0 : -1;                 // -1 but for the speaker row
+            for (int k = 0; k < W; ++k) h.ids[er * W + k] = 0;                     // the row's ids are unused
+            for (int t = 0; t < T; ++t) h.emb_map[t] = t == er ? 0 : -1;           // -1 but for the speaker row
             HIPX(hipMemcpyAsync(ctx->d_emb, sp.data(), (size_t) ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
         }
-        if (int rc = upload_inputs(ctx, er >= 0 ? (2 + W) * TM + T : 2 * TM + (size_t) T * W)) return rc;
-        if (int rc = run_step(ctx, T, h_np, ctx->d_slot, ctx->d_npast, ctx->d_ids, er >= 0 ? ctx->d_emb : nullptr,
-                              ctx->logits, /*kv_pre=*/true, er >= 0 ? ctx->d_emb_map : nullptr, h_slot, /*f32_prompt=*/true,
+        if (int rc = upload_inputs(ctx, (size_t) T * (er >= 0 ? 3 + W : 2 + W))) return rc;
+        if (int rc = run_step(ctx, T, h.n_past, d.slot, d.n_past, d.ids, er >= 0 ? ctx->d_emb : nullptr,
+                              ctx->logits, /*kv_pre=*/true, er >= 0 ? d.emb_map : nullptr, h.slot, /*f32_prompt=*/true,
                               last ? HEAD_LAST : HEAD_NONE)) return rc;
         if (last) return finish_pass(ctx, last_logits, row);
         HIPX(hipStreamSynchronize(ctx->stream));               // the pinned inputs are reused by the next chunk
@@ -2066,23 +2073,22 @@ int z2h_step_mixed(z2h_ctx * ctx, int n_rows, const int32_t * slot_idx, const in
     if (emb_map && (size_t) n_emb * ctx->hp.n_embd > (size_t) ctx->Tmax * ctx->hp.n_embd) return seterr(ctx, Z2H_EINVAL, "too many embedding rows");
     HIPX(hipSetDevice(ctx->device));
     ctx->resident_T = ctx->resident_last = 0;
-    const size_t TM = ctx->Tmax;
-    int32_t * h_slot = ctx->h_pin, * h_np = h_slot + TM, * hid = h_np + TM, * map = hid + TM * W, * hrows = map + TM;
-    std::memcpy(h_slot, slot_idx, (size_t) n_rows * 4);
-    std::memcpy(h_np, n_past, (size_t) n_rows * 4);
-    std::memcpy(hid, ids, (size_t) n_rows * W * 4);
-    for (int t = 0; emb_map && t < n_rows; ++t) {
-        map[t] = emb_map[t];
-        if (map[t] >= 0) for (int k = 0; k < W; ++k) hid[(size_t) t * W + k] = 0;     // unused ids
+    const PassInputs h = pass_inputs(ctx->h_pin, n_rows, W), d = pass_inputs(ctx->d_slot, n_rows, W);
+    std::memcpy(h.slot, slot_idx, (size_t) n_rows * 4);
+    std::memcpy(h.n_past, n_past, (size_t) n_rows * 4);
+    std::memcpy(h.ids, ids, (size_t) n_rows * W * 4);
+    for (int t = 0; t < n_rows; ++t) {                               // (without a map its ints are sent but not read)
+        h.emb_map[t] = emb_map ? emb_map[t] : -1;
+        if (h.emb_map[t] >= 0) for (int k = 0; k < W; ++k) h.ids[(size_t) t * W + k] = 0;     // unused ids
     }
-    if (n_out > 0) std::memcpy(hrows, out_rows, (size_t) n_out * 4);
-    if (int rc = upload_inputs(ctx, n_out > 0 ? (3 + W) * TM + n_out : emb_map ? (2 + W) * TM + n_rows : 2 * TM + (size_t) n_rows * W)) return rc;
+    if (n_out > 0) std::memcpy(h.head_rows, out_rows, (size_t) n_out * 4);
+    if (int rc = upload_inputs(ctx, (size_t) n_rows * (3 + W) + n_out)) return rc;
     if (emb_map) HIPX(hipMemcpyAsync(ctx->d_emb, emb, (size_t) n_emb * ctx->hp.n_embd * 4, hipMemcpyHostToDevice, ctx->stream));
     // every row appends its K/V before the attention; a slot's rows attend causally to each other; the
     // head runs on the requested rows only
-    if (int rc = run_step(ctx, n_rows, h_np, ctx->d_slot, ctx->d_npast, ctx->d_ids, emb_map ? ctx->d_emb : nullptr,
-                          ctx->logits, /*kv_pre=*/true, emb_map ? ctx->d_emb_map : nullptr, h_slot, false,
-                          HEAD_ROWS, ctx->d_head_rows, n_out)) return rc;
+    if (int rc = run_step(ctx, n_rows, h.n_past, d.slot, d.n_past, d.ids, emb_map ? ctx->d_emb : nullptr,
+                          ctx->logits, /*kv_pre=*/true, emb_map ? d.emb_map : nullptr, h.slot, false,
+                          HEAD_ROWS, d.head_rows, n_out)) return rc;
     return finish_pass(ctx, out_logits, (size_t) n_out * ctx->hp.n_codebooks * ctx->hp.audio_vocab);
 }
 
