@@ -106,3 +106,29 @@ def test_prefill_gemm_equals_narrow_passes(bulk, T):
         np.testing.assert_array_equal(a[0], b[0])
         np.testing.assert_array_equal(a[1], b[1])
     m.close()
+
+
+@pytest.mark.parametrize("T", [1037, 1080])
+@pytest.mark.parametrize("bulk", [Q8, Q6], ids=["q8_0", "q6_k"])
+def test_tall_tiles_equal_narrow_passes(bulk, T):
+    """matrices of 2048 rows, where a pass of this length takes the tallest token tiles (32 rows for Q8_0, 64 for Q6_K) in
+    W_o, the dense SwiGLU and down matmuls, and the experts'; the last tile is partly empty"""
+    cfg = configs.ModelConfig(f"tall-{bulk}", n_layer=3, n_embd=2048, n_head=8, n_head_kv=2, head_dim=64, n_expert=2, top_k=2, n_ff=2048,
+                              bulk=bulk, audio_vocab=33, expert_used=[0, 2, 0], router_mlp_std=0.1, router_out_std=0.2)
+    m = Model(cfg.hparams(), synth.generate_model(cfg, 8))
+    rng = np.random.default_rng(T)
+    ids = np.concatenate([rng.integers(0, cfg.audio_vocab, (T, cfg.n_codebooks)),
+                          rng.integers(0, cfg.text_vocab + 1, (T, 1))], axis=1).astype(np.int32)
+    outs, kvs = [], []
+    for chunk in (T, 16):
+        ctx = Context(None, 1, T, model=m, max_rows=T)
+        ctx.set_prefill_chunk(chunk)
+        print(f"{cfg.name}: {T} rows in passes of {chunk}", flush=True)
+        outs.append(ctx.prefill(0, ids))
+        kvs.append([ctx.kv_read(L, 0, 0, T) for L in range(cfg.n_layer)])
+        ctx.close()
+    for a, b in zip(*kvs):
+        np.testing.assert_array_equal(a[0], b[0])
+        np.testing.assert_array_equal(a[1], b[1])
+    np.testing.assert_array_equal(outs[0], outs[1])
+    m.close()

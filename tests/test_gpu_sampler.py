@@ -197,3 +197,39 @@ def test_resident_steps_stop_at_slot_capacity():
     # the context stays usable: a host step at valid rows runs
     c.step(slots, np.full(n, 5, np.int32), ids=ids)
     c.close()
+
+
+@pytest.mark.parametrize("av", [33, 256, 257, 1000, 2049, 4096])
+def test_device_sampler_vocabularies(av):
+    """Every width of the register sort (256 to 4096 entries), vocabularies that fill it and that leave most of it
+    to pads: distinct logits, tied ones, and ids masked by -inf or by the lowest float."""
+    import torch
+    n = 4
+    cfg = configs.ModelConfig(f"frames-{av}", n_layer=1, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_expert=0, top_k=0,
+                              n_ff=256, bulk=configs.F16, audio_vocab=av, expert_used=[0])
+    c = Context(cfg.hparams(), n, 16)
+    c.upload(synth.generate_model(cfg, 3))
+    ncb = cfg.n_codebooks
+    rng = np.random.default_rng(av)
+    settings = SETTINGS + [dict(temperature=1.0, top_k=1, top_p=0.0, min_p=0.0, rep_penalty=1.0, rep_codebooks=0, greedy=0),
+                           dict(temperature=0.7, top_k=av - 1, top_p=0.6, min_p=0.0, rep_penalty=1.3, rep_codebooks=9, greedy=0)]
+    for trial in range(18):
+        print(f"vocabulary {av}, trial {trial}", flush=True)
+        lg = rng.standard_normal((n, ncb, av)) * 2.5
+        if trial % 3 == 1:
+            lg = np.round(lg) * 0.5
+        lg = lg.astype(np.float32)
+        if trial % 3 == 2:
+            mask = rng.random((n, ncb, av)) < 0.5
+            mask[..., trial] = False
+            lg[mask] = (-np.inf, np.finfo(np.float32).min)[trial // 3 % 2]
+        sp = [settings[(trial + i) % len(settings)] for i in range(n)]
+        hist = rng.integers(0, av, (n, ncb, 64)).astype(np.int32)
+        hist[..., ::5] = trial
+        hlen = rng.integers(0, 65, (n, ncb)).astype(np.int32)
+        u = rng.random((n, ncb))
+        d = torch.from_numpy(lg).cuda()
+        torch.cuda.synchronize()
+        got = c.sample(sp, u, hist, hlen, d_logits=d.data_ptr())
+        np.testing.assert_array_equal(got, _oracle_codes(lg, sp, u, hist, hlen, 1))
+    c.close()
