@@ -3159,7 +3159,7 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
     // can hold another id. So the first pass flags the cases where an equal-key neighbour could swap
     // the outcome: a top-p cut inside a run of equal probabilities, a fallback whose top probability
     // is shared, or a code whose logit is shared (top-k). Those cases run again on the library's
-    // exact orders (z2h_order, one thread). The wave's lanes decide together; every lane has the answer.
+    // exact orders (z2h_order). The wave's lanes decide together; every lane has the answer.
     const double top_p = sp.top_p > 0.0f && sp.top_p < 1.0f ? (double) sp.top_p : -1.0;
     auto decide = [&](auto cand_at, auto rank_at, bool flag_ties, bool & tie) -> int {
         tie = false;
@@ -3199,16 +3199,21 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs a) {
         // the library's orders: ids by logit (std::partial_sort over all ids, first top_k kept), then
         // candidate positions by probability (std::sort); s_key is free now and holds the id arrays
         int * ord = (int *) s_key;
+        // (all lanes run the same steps on the same values; a comparison read from the first lane makes every branch
+        // and index uniform: a call of 64 columns of tied logits over 1026 ids, top-k 100: 788 us by one lane, 581 so)
+        auto uni = [](bool b) { return __builtin_amdgcn_readfirstlane((int) b) != 0; };
         wave_lds_sync();
-        if (lane == 0) {
-            if (topk) {
-                for (int i = 0; i < av; ++i) ord[i] = i;
-                z2h_order::partial_order(ord, n, av, [&](int x, int y) { return s_lg[x] > s_lg[y]; });
-                for (int j = 0; j < n; ++j) s_idx[j] = ord[j];
-            }
-            for (int j = 0; j < n; ++j) { ord[j] = j; s_keep[j] = 1; }
-            z2h_order::sort_order(ord, n, [&](int x, int y) { return s_p[x] > s_p[y]; });
+        if (topk) {
+            for (int i = lane; i < av; i += 64) ord[i] = i;
+            wave_lds_sync();
+            z2h_order::partial_order(ord, n, av, [&](int x, int y) { return uni(s_lg[x] > s_lg[y]); });
+            wave_lds_sync();
+            for (int j = lane; j < n; j += 64) s_idx[j] = ord[j];
+            wave_lds_sync();
         }
+        for (int j = lane; j < n; j += 64) { ord[j] = j; s_keep[j] = 1; }
+        wave_lds_sync();
+        z2h_order::sort_order(ord, n, [&](int x, int y) { return uni(s_p[x] > s_p[y]); });
         wave_lds_sync();
         code = decide([&](int j) { return topk ? s_idx[j] : j; }, [&](int r) { return ord[r]; }, false, tie);
     }
