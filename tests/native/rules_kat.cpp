@@ -5,11 +5,12 @@
 
 int main() {
     char what[32];
-    long long a, b, c, d;
-    while (std::scanf("%31s %lld %lld %lld %lld", what, &a, &b, &c, &d) == 5) {
+    long long a, b, c, d, e;
+    while (std::scanf("%31s %lld %lld %lld %lld %lld", what, &a, &b, &c, &d, &e) == 6) {
         if (!std::strcmp(what, "tall")) std::printf("%d\n", (int) z2r::f16_tall_tiles(a, b, (int) c, (int) d));
         else if (!std::strcmp(what, "few")) std::printf("%d\n", (int) z2r::f16_few_rows(a, (int) b, (int) c));
         else if (!std::strcmp(what, "rdown")) std::printf("%d\n", (int) z2r::router_down_reuse((int) a, (int) b, c != 0));
+        else if (!std::strcmp(what, "qexp")) std::printf("%d\n", (int) z2r::quant_gemm_experts(a != 0, b, (int) c, d, e));
         else return 1;
     }
     return 0;

@@ -13,7 +13,7 @@ def ask(root, tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", str(root / "tests" / "native" / "rules_kat.cpp"), "-o", str(exe)], check=True)
 
     def run(queries):
-        text = "\n".join(" ".join(map(str, q)) for q in queries)
+        text = "\n".join(" ".join(map(str, (*q, 0, 0, 0, 0)[:6])) for q in queries)
         out = subprocess.run([str(exe)], input=text, check=True, capture_output=True, text=True).stdout.split()
         assert len(out) == len(queries)
         return [x == "1" for x in out]
@@ -73,3 +73,15 @@ RDOWN = [((65, 768), False), ((200, 768), True), ((65, 1024), False), ((160, 102
 def test_router_down_reuse(ask):
     full = lambda d: d % 64 == 0 and d // 64 & (d // 64 - 1) == 0
     assert ask([("rdown", T, d, int(full(d)), 0) for (T, d), _ in RDOWN]) == [w for _, w in RDOWN]
+
+
+# (Q6_K, routes, experts, model width, FFN width) -> the GEMMs
+QEXP = [((0, 72, 8, 512, 256), False), ((0, 384, 8, 512, 256), False), ((0, 800, 8, 512, 256), True), ((0, 192, 16, 1024, 768), False),
+        ((0, 512, 8, 1024, 768), True), ((0, 256, 32, 2048, 1536), True), ((0, 255, 32, 2048, 1536), False), ((0, 64, 4, 2048, 1536), False),
+        ((0, 256, 4, 2048, 1536), True), ((0, 1025, 128, 512, 256), True), ((0, 1025, 129, 512, 256), False),
+        ((1, 72, 8, 512, 256), False), ((1, 384, 8, 512, 256), True), ((1, 72, 8, 1024, 768), False), ((1, 160, 8, 1024, 768), True),
+        ((1, 72, 4, 2048, 1536), True), ((1, 255, 32, 2048, 1536), False)]
+
+
+def test_quant_gemm_experts(ask):
+    assert ask([("qexp", q6, r, E, d * ff, 1024) for (q6, r, E, d, ff), _ in QEXP]) == [w for _, w in QEXP]

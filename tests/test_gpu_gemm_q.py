@@ -1,6 +1,6 @@
 """The Q8_0 and Q6_K GEMMs of wide passes (k_gemm_q80, k_gemm_q6k) against the GEMVs of narrow ones: an
 MoE layer over T rows gives the same bits as the same rows in calls of at most 16 (which take the
-GEMVs), at token tiles of every height and their remainders, at rows and K that do not fill the blocks,
+GEMVs; so do the shorter of the others, where the GEMMs do not pay), at token tiles of every height and their remainders, at rows and K that do not fill the blocks,
 and with activations whose block scales are f16 subnormals or large. A prompt prefilled in one pass
 (dense projections and dense FFN as GEMMs) gives the bits of 16-row passes. The GEMVs are held to the
 oracle elsewhere; one layer here is too."""
@@ -26,7 +26,8 @@ def _cfg(bulk, E, k, ff, d=512, dense=0):
 
 @pytest.mark.parametrize("scale", [1.0, 1e-5, 1e5], ids=["x1", "x1e-5", "x1e5"])
 @pytest.mark.parametrize("bulk,E,k,ff,T", [(Q8, 8, 2, 288, 67), (Q8, 4, 2, 288, 17), (Q8, 4, 1, 256, 300), (Q8, 2, 2, 800, 1501),
-                                           (Q6, 8, 2, 256, 67), (Q6, 4, 2, 512, 17), (Q6, 4, 1, 256, 300), (Q6, 2, 2, 768, 1501)])
+                                           (Q6, 8, 2, 256, 67), (Q6, 4, 2, 512, 17), (Q6, 4, 1, 256, 300), (Q6, 2, 2, 768, 1501),
+                                           (Q8, 8, 2, 288, 325), (Q8, 64, 1, 288, 650), (Q8, 3, 1, 544, 647), (Q6, 8, 2, 256, 170), (Q6, 64, 1, 256, 650), (Q6, 3, 1, 512, 331)])
 def test_moe_gemm_equals_gemv(bulk, E, k, ff, T, scale):
     cfg = _cfg(bulk, E, k, ff)
     m = Model(cfg.hparams(), synth.generate_model(cfg, 5 + T))
@@ -54,7 +55,7 @@ def test_non_finite_scales_stay_in_their_block(bulk, offset, f16):
         raw[row * rb + blk * bb + offset:][:2] = np.frombuffer(np.uint16(f16).tobytes(), np.uint8)
     model["blk.0.ffn_down_exps.weight"] = dataclasses.replace(t, data=raw)
     m = Model(cfg.hparams(), model)
-    T = 67
+    T = 331
     ctx = Context(None, 1, 256, model=m, max_rows=T)
     x = np.random.default_rng(2).standard_normal((T, cfg.n_embd)).astype(np.float32)
     x[3] *= 1e9                                                          # its block scales are infinite in f16
@@ -70,13 +71,13 @@ def test_non_finite_scales_stay_in_their_block(bulk, offset, f16):
 
 
 @pytest.mark.parametrize("bulk", [Q8, Q6], ids=["q8_0", "q6_k"])
-def test_moe_gemm_vs_oracle(bulk):
+@pytest.mark.parametrize("T", [131, 331])
+def test_moe_gemm_vs_oracle(bulk, T):
     cfg = _cfg(bulk, 4, 2, 256)
     model = synth.generate_model(cfg, 9)
-    ctx = Context(cfg.hparams(), 1, 256, max_rows=131)
-    ctx.upload(model)
+    ctx = Context(None, 1, 256, model=Model(cfg.hparams(), model), max_rows=T)
     om = O.OracleModel(cfg.hparams(), model)
-    x = np.random.default_rng(3).standard_normal((131, cfg.n_embd)).astype(np.float32)
+    x = np.random.default_rng(3).standard_normal((T, cfg.n_embd)).astype(np.float32)
     print(f"{cfg.name} vs oracle", flush=True)
     got = ctx.moe_forward(0, x)
     ref = O.router(om, 0, x, None)

@@ -629,10 +629,8 @@ int cap_copy(z2h_ctx * ctx, int what, int L, const void * src, int T) {
 //                K-split GEMV's four times as many blocks win (48 rows of QKV, 147 blocks: 8.0 us against 10.5
 //                for Q8_0; 64 rows of W_o, 128 blocks: 8.0 against 6.5; the 9225-row
 //                Q8_0 head of 5 rows 8.8 against 10.1, of 16 rows 9.7 against 12.5, of 64 rows 17.6 against
-//                27.4). One and two rows keep the token-pair units. Experts: at least 8 routes per expert
-//                on average, where the GEMV starts re-reading its weights per 8- or 16-route pass (64 rows,
-//                top-4 of 32: Q6_K gate/up 38 us against 52, down 22 against 32; 48 rows, 6 routes: level
-//                before the sort launch is counted). Q8_0 matrices with an infinite or NaN block scale stay on
+//                27.4). One and two rows keep the token-pair units. Experts:
+//                quant_gemm_experts. Q8_0 matrices with an infinite or NaN block scale stay on
 //                the GEMVs at every width: k_gemm_q80 multiplies a row's other scales of the superblock by zero.
 constexpr int GEMM_MIN_ROWS = 65;
 // (k_gemm_q4k's activation offsets are 32-bit)
@@ -645,7 +643,7 @@ bool use_gemm(const z2h_ctx * ctx, const DevMat & m, int n_tok) {
 bool use_gemm_experts(const DevMat & m, int n_tok, int k, int E) {
     if (!m.m16) return m.type == Z2H_F16;
     if (m.type == Z2H_Q4_K) return n_tok >= GEMM_MIN_ROWS && gemm_q4k_ok(m, (int64_t) n_tok * k);
-    return m.finite && n_tok > MT && (int64_t) n_tok * k >= 8ll * E;
+    return m.finite && n_tok > MT && z2r::quant_gemm_experts(m.type == Z2H_Q6_K, (int64_t) n_tok * k, E, (int64_t) m.rows * m.K, LIST_MAX);
 }
 // gate and up fused with SwiGLU in one GEMM launch: same type, layout and shape
 bool gemm_dual_ok(const DevMat & g, const DevMat & u) {

@@ -40,6 +40,21 @@ inline bool f16_few_rows(int64_t rows, int nsb, int n_tok) {
     return nsb >= 2 && rows <= 4096ll * nsb && (nsb > 2 || n_tok <= 32);
 }
 
+// Q8_0 and Q6_K expert matmuls: the GEMMs instead of the GEMVs. From 8 routes per expert on average the GEMV reads its weights
+// again for every 8 or 16 routes of an expert. A launch whose routes the GEMV blocks could list by themselves (`list` at
+// most) pays another launch of about 4 us for the GEMM, the route sort: there the line follows the work saved, which grows with
+// the routes and the weights of an expert (`elems` per matrix). Whole MoE layer calls, us, GEMV / GEMM, by routes:
+//   Q8_0  512 x 256, 8 experts: 72 38.8 / 42.2, 512 42.8 / 43.8, 800 51.1 / 46.1; 1024 x 768, 16 experts: 192 47.6 / 49.1, 320
+//         55.1 / 52.4; 2048 x 1536, 32 experts: 256 91.3 / 92.9 (Zipf 1.2: 78 / 62), 288 99.1 / 95.5; 4 experts: 64
+//         48.1 / 49.0, 256 60.5 / 59.7; 16 experts: 256 65.5 / 68.9, 320 73.2 / 69.3
+//   Q6_K  512 x 256, 8 experts: 72 40.0 / 42.6, 384 44.6 / 43.4; 1024 x 768, 8 experts: 72 45.0 / 46.9, 160 51.0 / 50.3;
+//         2048 x 1536, 32 experts: 256 105 / 85; 4 experts: 64 56.4 / 53.5
+inline bool quant_gemm_experts(bool q6_k, int64_t routes, int E, int64_t elems, int64_t list) {
+    if (routes < 8ll * E) return false;
+    const double work = (double) routes * (double) routes * (double) elems;
+    return routes > list || (q6_k ? work >= 1.3e10 : routes >= 640 || work >= 1.6e11);
+}
+
 // The router down projection alone (an MoE layer call): k_router_down_t, which loads a weight row once for many tokens, instead
 // of k_router_down's block per token and four outputs. Up to 512 columns it is never the slower one; above, it pays from
 // about the work of 65 rows of 2048 columns, and rows of more than 2048 columns that leave part of the last chain step
