@@ -177,7 +177,7 @@ def decode_leg(np, torch, cfg, wl, steps, warmup, cpu_steps, label, keep=False):
         "cfg": cfg, "wl": wl, "T": T, "ms": ms, "med_ms": med_ms, "host_med": host_med, "prof": prof, "B": B,
         "step_gbps": step_gbps, "dom_gbps": dom_gbps, "gu_ms": gu_ms, "gu_n": gu_n,
         "gu_bytes": int((gu_w + act_b + gu_out) / max(1, len(moe))),
-        "roofline": {"kernel": gateup_kernel_of(cfg.bulk), "bound": "hbm", "achieved": round(dom_gbps, 1),
+        "roofline": {"kernel": gateup_kernel_of(cfg, T), "bound": "hbm", "achieved": round(dom_gbps, 1),
                      "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(dom_gbps / HBM_PEAK_GBPS, 4),
                      "avg_launch_us": round(gu_ms / max(1, gu_n) * 1000.0, 2),
                      "bytes_per_launch": int((gu_w + act_b + gu_out) / max(1, len(moe)))},
@@ -536,9 +536,13 @@ def type_name(t):
     return TYPE_NAMES[t]
 
 
-def gateup_kernel_of(bulk):
+def gateup_kernel_of(cfg, n):
+    """the grouped gate/up kernel of an n-request step of the 24-layer configurations (up to 64 requests, experts of
+    2048 x 1536): the GEMMs take Q8_0 and Q6_K from 8 routes per expert on (csrc/z2h_rules.h)"""
     from zonos2_amd.configs import TYPE_NAMES
-    w = TYPE_NAMES[bulk]
+    w = TYPE_NAMES[cfg.bulk]
+    if w in ("Q8_0", "Q6_K") and n * cfg.top_k >= 8 * cfg.n_expert:
+        return f"k_gemm_{'q80' if w == 'Q8_0' else 'q6k'}<DUAL> grouped expert gate/up + SwiGLU"
     if w in ("Q4_K", "Q8_0", "Q6_K"):
         return f"k_gemv_mfma<{w}, DUAL> grouped expert gate/up + SwiGLU"
     return f"k_gemm_f16<DUAL> grouped expert gate/up + SwiGLU"

@@ -17,7 +17,7 @@
 //                fold of the Q4_K GEMVs, so a row's result is the same bits at any batch width.
 //   k_gemm_f16   F16 weights (t64 layout) x f16 activations on v_mfma_f32_16x16x32_f16, fp32
 //                accumulation; the weight fragments stream straight from HBM into a register ring of
-//                32-column steps. Every F16 matmul (decode widths too) runs on it.
+//                32-column steps. Decode widths run on its narrow shape, or on k_gemm_f16_few.
 #pragma once
 #include "z2h_kernels.h"
 
@@ -129,8 +129,8 @@ __device__ __forceinline__ void gemm_store(const GemmArgs & a, const float (&acc
 // token rows. The wave's 32 rows are one B operand of v_mfma_i32_32x32x32_i8: lane l has row l % 32
 // (16-row group (l / 16) & 1; DUAL: gate, up) and columns 32 j + 16 h .. + 15 of sub-block j, h = l / 32.
 //
-// Bounded by issue, not by memory (L2 hits at 80%, HBM idle): the vector unit (the weights' unpacking, 22
-// instructions per sub-block, and the fp32 fold, 5 per output) and the matrix unit are busy 60% and 34%
+// Bounded by issue, not by memory (82% of the L2 reads hit): the vector unit (the weights' unpacking, 22
+// instructions per sub-block, and the fp32 fold, 5 per output) and the matrix unit are busy 57% and 32%
 // of the time. So the unpacking of sub-block j + 1 sits between the products of sub-block j (the group
 // barriers), 32 x 32 products take half the LDS reads and min-term products of 16 x 16 ones, the min term
 // takes the sums of 16 as they are, the staging has no address arithmetic, and a SwiGLU is formed once per output

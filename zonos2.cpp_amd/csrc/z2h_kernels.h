@@ -357,7 +357,7 @@ __device__ __forceinline__ float4 table_elem4_t(const uint8_t * row, int i0) {
 // last barrier (a barrier waits for the block's outstanding stores). One instantiation per mode
 // keeps each kernel's code to its own path. TT >= 0 (RN_EMBED): every table has GGUF type TT, and the
 // token's table rows are read with no type switch: all tables' loads of an element group go out
-// together (TW table slots, W <= TW; slots past W re-read the last table and are not added), the sum
+// together (TW table slots, W <= TW; slots past W re-read the first table and are not added), the sum
 // keeps the table order.
 constexpr int RN_NV = 4;
 template <int MODE, int TT = -1, int TW = MAX_TABLES>
