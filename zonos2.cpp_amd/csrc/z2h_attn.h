@@ -532,10 +532,10 @@ __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
     }
     FH_LOAD(0)
     // ---- queries (wave w: row-heads w, w + 8, ...; per-head RMSNorm, |temp|, RoPE; f16 for the products)
-    {
+    auto form = [&](auto count) {
         // every input (the RoPE pairs from the per-position table) is loaded before the arithmetic, and all row-heads
         // are formed without branches, so that their reductions overlap (row-heads past P repeat the last)
-        constexpr int QW = 8;
+        constexpr int QW = decltype(count)::value;
         float2 xq[QW], cq[QW];
         float mul[QW];
 #pragma unroll
@@ -555,7 +555,11 @@ __global__ void __launch_bounds__(512) k_attn_flash16(AttnArgs a) {
             *(float2 *) &s_q[rq * (HD + 4) + 2 * lane] = y[k];
             if (a.cap_q) *(float2 *) (a.cap_q + ((int64_t) (t0 + rq / GRP) * a.nh + g * GRP + rq % GRP) * HD + 2 * lane) = y[k];
         }
-    }
+    };
+    // (a decode column's tile has one row, one row-head per wave; a full tile 16 GRP. 65 columns of a mixed pass, 16 heads,
+    // with eight of them in each wave for every tile: 7.2 us without cached rows, 10.3 with 300; so 5.6 and 9.4)
+    if (__builtin_amdgcn_readfirstlane(P) <= 8) form(std::integral_constant<int, 1>{});
+    else form(std::integral_constant<int, 2 * GRP>{});
     lds_sync();
     const int rh = 16 * wq + c16;                                    // the lane's row-head (B columns)
     const bool rh_ok = rh < P;
@@ -763,7 +767,7 @@ __global__ void __launch_bounds__(512) k_attn_flash32(AttnArgs a) {
     {
         // every input (the RoPE pairs from the per-position table) is loaded before the arithmetic, and all row-heads
         // are formed without branches, so that their reductions overlap (row-heads past P repeat the last)
-        constexpr int QW = 8;
+        constexpr int QW = 2 * GRP;                                  // (16 GRP row-heads over 8 waves)
         float2 xq[QW], cq[QW];
         float mul[QW];
 #pragma unroll
