@@ -71,14 +71,30 @@ def test_non_finite_scales_stay_in_their_block(bulk, offset, f16):
 
 
 @pytest.mark.parametrize("bulk", [Q8, Q6], ids=["q8_0", "q6_k"])
-@pytest.mark.parametrize("T", [131, 331])
-def test_moe_gemm_vs_oracle(bulk, T):
+def test_moe_gemm_vs_oracle(bulk):
     cfg = _cfg(bulk, 4, 2, 256)
     model = synth.generate_model(cfg, 9)
-    ctx = Context(None, 1, 256, model=Model(cfg.hparams(), model), max_rows=T)
+    ctx = Context(cfg.hparams(), 1, 256, max_rows=131)
+    ctx.upload(model)
     om = O.OracleModel(cfg.hparams(), model)
-    x = np.random.default_rng(3).standard_normal((T, cfg.n_embd)).astype(np.float32)
+    x = np.random.default_rng(3).standard_normal((131, cfg.n_embd)).astype(np.float32)
     print(f"{cfg.name} vs oracle", flush=True)
+    got = ctx.moe_forward(0, x)
+    ref = O.router(om, 0, x, None)
+    _, want = O.experts(om, 0, x, ref["sel"], ref["w"])
+    assert_close(cfg.name, got, want)
+    ctx.close()
+
+
+@pytest.mark.parametrize("bulk", [Q8, Q6], ids=["q8_0", "q6_k"])
+def test_moe_gemm_of_many_rows_vs_oracle(bulk):
+    """(331 rows: above the line from which layers of this size take the GEMMs)"""
+    cfg = _cfg(bulk, 4, 2, 256)
+    model = synth.generate_model(cfg, 9)
+    ctx = Context(None, 1, 256, model=Model(cfg.hparams(), model), max_rows=331)
+    om = O.OracleModel(cfg.hparams(), model)
+    x = np.random.default_rng(3).standard_normal((331, cfg.n_embd)).astype(np.float32)
+    print(f"{cfg.name}, {len(x)} rows vs oracle", flush=True)
     got = ctx.moe_forward(0, x)
     ref = O.router(om, 0, x, None)
     _, want = O.experts(om, 0, x, ref["sel"], ref["w"])
